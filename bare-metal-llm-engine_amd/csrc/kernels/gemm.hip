@@ -1,20 +1,22 @@
-// gemm.hip -- FP32 GEMM on gfx950 matrix cores (C[M x N] = A[M x K] . B[K x N]).
+// gemm.hip -- the GEMMs (C[M x N] = A[M x K] . B).
 //
 // Replaces the SIMT register-tiled kernel behind matmul_register_tiled
-// (reference kernels/matmul_register_tiled.cu:48-199); it is also the M > 1
-// half of rmsnorm_linear, which, as in the reference
-// (kernels/rmsnorm_linear.cu:191-199), normalises the rows into scratch
-// first. (Fusing the RMSNorm into this kernel -- gamma applied to the A
-// fragments, row sums of squares taken from them -- measured 30% slower than
-// the separate pass at 512 x 4096 x 4096: every N-tile repeats the multiply,
-// and it sits between the LDS read and the MFMA.)
+// (reference kernels/matmul_register_tiled.cu:48-199); also the M > 1 half of
+// rmsnorm_linear, which, as in the reference (kernels/rmsnorm_linear.cu:191-199),
+// normalises the rows into scratch first. (Fusing the RMSNorm into the FP32
+// kernel -- gamma applied to the A fragments, row sums of squares taken from
+// them -- measured 30% slower than the separate pass at 512 x 4096 x 4096.)
 //
-// Tiling for wave64 and v_mfma_f32_32x32x2_f32:
-//   * workgroup tile BM x BN (256 x 128, 128 x 128, 128 x 64 or 64 x 64), K
-//     step 32; 256 x 128 runs 512 threads = 8 waves in 4 x 2 with three LDS
-//     stages, one workgroup per CU, the others 256 threads = 4 waves in 2 x 2
-//     with two stages, two workgroups per CU; each wave owns its block of the
-//     tile as 32 x 32 MFMA blocks;
+//   * fp32 B, and fp16 B where the next item does not apply: gemm_split.hip, on
+//     the bf16 matrix cores; here the FP32-instruction kernels it leaves the
+//     small calls to: gemm_small_splitk_kernel (up to half a round of 64 x 64
+//     tiles) and gemm_f32_mfma_dma_kernel (64 x 64 tiles, about one round);
+//   * fp16 B against activations split into three fp16 planes:
+//     gemm_h3_kernel / gemm_h3_sk_kernel.
+//
+// gemm_f32_mfma_dma_kernel, for wave64 and v_mfma_f32_32x32x2_f32:
+//   * 64 x 64 tiles, K step 32, 4 waves of 32 x 32, two LDS stages, two
+//     workgroups per CU;
 //   * operand layout of the instruction: lane l supplies A[l % 32][k] and
 //     B[k][l % 32] with k = l / 32 of the pair; accumulator v of lane l is
 //     C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32]. Within a 32-deep K tile the
@@ -22,24 +24,15 @@
 //     32-63), so each lane reads a contiguous 16-float run of its A row
 //     (ds_read_b128) and a 16-row column of B (ds_read_b32, conflict-free) --
 //     or, when B is given transposed ([N x K]), a 16-float run of its B row;
-//   * operands with K % 32 == 0 and 16-byte aligned rows take
-//     gemm_f32_mfma_dma_kernel, which loads tiles straight into LDS (below;
-//     fp16 B is converted as fragments are read; ragged M / N clamp their edge
-//     loads); the rest take gemm_f32_mfma_kernel, which stages through registers: A and B tiles are
-//     double-buffered in LDS with 4-float row padding and the next tile's
-//     global loads are issued before the current tile's MFMAs;
-//   * the workgroup -> tile map is XCD-aware: consecutive workgroup ids go to
-//     different XCDs, so ids are regrouped so each XCD works on a contiguous
-//     band of tiles (grouped 8 tile-rows deep) and shares A/B panels in its L2;
-//   * the tile shape is chosen per call so the grid covers the 256 CUs evenly
-//     (small-M shapes such as 512 x 4096 x 11008 would leave half the CUs idle
-//     with 128 x 128 tiles);
-//   * fragments are read a quarter K tile (4 MFMA k-slices) ahead of the
-//     MFMAs that use them.
+//   * fragments are read a quarter K tile (4 MFMA k-slices) ahead of the MFMAs
+//     that use them.
+// The workgroup -> tile map of every GEMM here is XCD-aware (tile_of).
+#include "gemm_plan.hpp"
 #include "launch.hpp"
 
 #include <algorithm>
 #include <cstdlib>
+#include <limits>
 #include <type_traits>
 
 namespace eng {
@@ -50,10 +43,92 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 
 constexpr int BK = 32;
-constexpr int kThreads = 256;
-constexpr int AS = BK + 4;   // row stride (floats) of k-contiguous tiles in LDS
-constexpr int kGroupM = 8;   // tile-rows per raster group
-constexpr int kXcds = 8;
+// Direct global -> LDS loads (buffer_load_dwordx4 ... lds:
+// lane l of a wave writes 16 bytes at the wave's LDS base + 16 l, from the
+// offset the lane names past the descriptor's base). No staging registers and
+// no LDS store instructions: a stage's loads are issued one or two K tiles
+// before it is read and land while the MFMAs run; one s_waitcnt and one
+// barrier hand each stage over. LDS tiles are unpadded and the 16-byte chunk
+// positions are XOR-swizzled instead, which the fetch side applies by choosing
+// which global chunk each lane loads:
+//   * k-contiguous tiles (A, and B given [N x K]): chunk c of row r sits at
+//     c ^ ((r >> 1) & 7), so the 16 rows a 16-lane slice of ds_read_b128
+//     touches fall in 16 distinct bank groups;
+//   * [K x N] B tiles: chunk c of row k sits at c ^ (8 ((k >> 4) & 1)), so the
+//     rows k and k + 16 read by the two half-waves of a ds_read_b32 use
+//     disjoint banks.
+// Requires K % 32 == 0 and 16-byte aligned A and B (ragged M / N: EDGE below).
+__device__ __forceinline__ int swz_rows(int r) { return (r >> 1) & 7; }
+
+// 16-byte direct load into LDS through a buffer descriptor: lane l reads the
+// bytes [off, off + 16) past base and writes them to lds + 16 l (lds the same
+// in every lane of the wave). The descriptor covers `bytes` bytes from base
+// (reads past them return zeros). base must be wave-uniform. Buffer loads,
+// unlike global_load_lds, are not FLAT instructions: the compiler then counts
+// the in-flight direct loads on vmcnt only and keeps the LDS fragment reads'
+// waits partial instead of draining them with lgkmcnt(0).
+[[maybe_unused]] constexpr int kRsrcWord3 = 0x00020000;  // gfx9 buffer descriptor word 3 (raw dword access)
+
+template <typename T>
+__device__ __forceinline__ void lds_buf16(const T* base, unsigned bytes, unsigned off, T* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, static_cast<int>(bytes), kRsrcWord3),
+      lds, 16, static_cast<int>(off), 0, 0, 0);
+#endif
+}
+
+// Bytes from element `from` to the end of an n-element array, capped at the
+// 32-bit range of a buffer descriptor.
+template <typename T>
+__device__ __forceinline__ unsigned bytes_left(long long n, long long from) {
+  const unsigned long long b = static_cast<unsigned long long>(n - from) * sizeof(T);
+  return (b >> 32) != 0 ? 0xFFFFFFFFu : static_cast<unsigned>(b);
+}
+
+// Waits until this wave's outstanding memory operations, the direct LDS loads
+// included, have completed.
+__device__ __forceinline__ void wait_all_memory() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_s_waitcnt(0);
+#endif
+}
+
+// Stage hand-over inside the K loop: waits until at most `vm` of this wave's
+// vector-memory operations (direct LDS loads, issued and completing in order)
+// are outstanding and all of its LDS reads have returned, then joins the
+// workgroup barrier. The barrier is the bare instruction rather than
+// __syncthreads(), whose release fence would drain every outstanding load
+// (vmcnt(0)) and so cap the ring at one tile in flight; the empty asm
+// statements keep the compiler from moving memory accesses across it.
+template <int VM>
+__device__ __forceinline__ void stage_barrier() {
+  static_assert(VM >= 0 && VM < 64, "vmcnt field");
+#if defined(__HIP_DEVICE_COMPILE__)
+  // gfx9 s_waitcnt: vmcnt bits 3:0 and 15:14, expcnt 6:4 (7 = no wait),
+  // lgkmcnt 11:8 (0 = wait for all)
+  __builtin_amdgcn_s_waitcnt((VM & 0xF) | ((VM >> 4) << 14) | (0x7 << 4));
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#endif
+}
+__device__ __forceinline__ int swz_kn(int k) { return ((k >> 4) & 1) * 8; }
+// fp16 [N x K] tiles (8 halves per 16-byte chunk): a 32-deep row is 4 chunks;
+// chunk c of row r sits at c ^ ((r >> 2) & 3), so the 16 rows of a 16-lane
+// slice of ds_read_b128 (row pitch 64 bytes) cover all 64 banks.
+__device__ __forceinline__ int swz_rows_h(int r) { return (r >> 2) & 3; }
+
+namespace f32 {
+constexpr int BM = 64;
+constexpr int BN = 64;
+constexpr int WGN = 2;                     // waves along N (and 2 along M)
+constexpr int kWaves = 4;
+constexpr int kThreads = 64 * kWaves;
+constexpr int INST = BM * BK / 4 / kThreads;  // direct loads per thread per operand tile
+}  // namespace f32
+
+constexpr int AS = BK + 4;  // row stride (floats) of k-contiguous register-staged tiles
 
 // Global -> register staging of a B tile: 16-byte vectors, `kLoads` per thread.
 // K x N layout: BK rows of BN elements; N x K layout: BN rows of BK elements.
@@ -62,36 +137,23 @@ struct BStage {
   static constexpr int kVec = 16 / static_cast<int>(sizeof(BT));
   static constexpr int kRowLen = BNK ? BK : BN;
   static constexpr int kThreadsPerRow = kRowLen / kVec;
-  static constexpr int kRowsPerLoad = kThreads / kThreadsPerRow;
+  static constexpr int kRowsPerLoad = f32::kThreads / kThreadsPerRow;
   static constexpr int kLoads = (BNK ? BN : BK) / kRowsPerLoad;
   static_assert(kLoads >= 1 && kLoads * kRowsPerLoad == (BNK ? BN : BK), "B staging shape");
 };
 
-// Workgroup id -> (tile_m, tile_n). Workgroups are handed to XCDs round-robin,
-// so id w runs on XCD w % 8; renumber so XCD x gets a contiguous logical range,
-// then raster that range in groups of kGroupM tile-rows.
-__device__ __forceinline__ void tile_of(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int ntiles = tiles_m * tiles_n;
-  const int q = ntiles / kXcds;
-  const int r = ntiles % kXcds;
-  const int xcd = wg % kXcds;
-  const int local = wg / kXcds;
-  const int logical = xcd * q + (xcd < r ? xcd : r) + local;
-  const int group_size = kGroupM * tiles_n;
-  const int group = logical / group_size;
-  const int first_m = group * kGroupM;
-  const int gm = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
-  const int in_group = logical - group * group_size;
-  tm = first_m + in_group % gm;
-  tn = in_group / gm;
-}
-
+// The FP32 instruction with tiles staged through registers (double-buffered in
+// LDS with 4-float row padding; fp16 B converted on the way): any K, N and
+// alignment. It keeps the short unaligned K that gemm_split.hip's longer
+// pipeline fill costs more than the sums (200 x 3001 x 64: 4.8 against 6.0 us).
 // BNK: B is given as B^T, row-major [N x K]; its tile is staged like an A
 // tile (n rows, k contiguous) and its fragments are read like A's.
-template <int BM, int BN, typename BT, bool BNK, bool VA, bool VB>
-__global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma_kernel(
+template <typename BT, bool BNK, bool VA, bool VB>
+__global__ __launch_bounds__(f32::kThreads, 2) void gemm_f32_mfma_kernel(
     const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ C, int M, int N,
     int K, int tiles_m, int tiles_n) {
+  constexpr int BM = f32::BM;
+  constexpr int BN = f32::BN;
   using BL = BStage<BT, BNK, BN>;
   constexpr int WM = BM / 2;       // rows per wave
   constexpr int WN = BN / 2;       // columns per wave
@@ -268,163 +330,36 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_mfma_kernel(
   }
 }
 
-// Variant fed by direct global -> LDS loads (buffer_load_dwordx4 ... lds:
-// lane l of a wave writes 16 bytes at the wave's LDS base + 16 l, from the
-// offset the lane names past the descriptor's base). No staging registers and
-// no LDS store instructions: a stage's loads are issued one or two K tiles
-// before it is read and land while the MFMAs run; one s_waitcnt and one
-// barrier hand each stage over. LDS tiles are unpadded and the 16-byte chunk
-// positions are XOR-swizzled instead, which the fetch side applies by choosing
-// which global chunk each lane loads:
-//   * k-contiguous tiles (A, and B given [N x K]): chunk c of row r sits at
-//     c ^ ((r >> 1) & 7), so the 16 rows a 16-lane slice of ds_read_b128
-//     touches fall in 16 distinct bank groups;
-//   * [K x N] B tiles: chunk c of row k sits at c ^ (8 ((k >> 4) & 1)), so the
-//     rows k and k + 16 read by the two half-waves of a ds_read_b32 use
-//     disjoint banks.
-// Requires K % 32 == 0 and 16-byte aligned A and B (ragged M / N: EDGE below).
-__device__ __forceinline__ int swz_rows(int r) { return (r >> 1) & 7; }
-
-// 16-byte direct load into LDS through a buffer descriptor: lane l reads the
-// bytes [off, off + 16) past base and writes them to lds + 16 l (lds the same
-// in every lane of the wave). The descriptor covers `bytes` bytes from base
-// (reads past them return zeros). base must be wave-uniform. Buffer loads,
-// unlike global_load_lds, are not FLAT instructions: the compiler then counts
-// the in-flight direct loads on vmcnt only and keeps the LDS fragment reads'
-// waits partial instead of draining them with lgkmcnt(0).
-[[maybe_unused]] constexpr int kRsrcWord3 = 0x00020000;  // gfx9 buffer descriptor word 3 (raw dword access)
-
-template <typename T>
-__device__ __forceinline__ void lds_buf16(const T* base, unsigned bytes, unsigned off, T* lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, static_cast<int>(bytes), kRsrcWord3),
-      lds, 16, static_cast<int>(off), 0, 0, 0);
-#endif
-}
-
-// Bytes from element `from` to the end of an n-element array, capped at the
-// 32-bit range of a buffer descriptor.
-template <typename T>
-__device__ __forceinline__ unsigned bytes_left(long long n, long long from) {
-  const unsigned long long b = static_cast<unsigned long long>(n - from) * sizeof(T);
-  return (b >> 32) != 0 ? 0xFFFFFFFFu : static_cast<unsigned>(b);
-}
-
-// Waits until this wave's outstanding memory operations, the direct LDS loads
-// included, have completed.
-__device__ __forceinline__ void wait_all_memory() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_s_waitcnt(0);
-#endif
-}
-
-// Stage hand-over inside the K loop: waits until at most `vm` of this wave's
-// vector-memory operations (direct LDS loads, issued and completing in order)
-// are outstanding and all of its LDS reads have returned, then joins the
-// workgroup barrier. The barrier is the bare instruction rather than
-// __syncthreads(), whose release fence would drain every outstanding load
-// (vmcnt(0)) and so cap the ring at one tile in flight; the empty asm
-// statements keep the compiler from moving memory accesses across it.
-template <int VM>
-__device__ __forceinline__ void stage_barrier() {
-  static_assert(VM >= 0 && VM < 64, "vmcnt field");
-#if defined(__HIP_DEVICE_COMPILE__)
-  // gfx9 s_waitcnt: vmcnt bits 3:0 and 15:14, expcnt 6:4 (7 = no wait),
-  // lgkmcnt 11:8 (0 = wait for all)
-  __builtin_amdgcn_s_waitcnt((VM & 0xF) | ((VM >> 4) << 14) | (0x7 << 4));
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-#endif
-}
-__device__ __forceinline__ int swz_kn(int k) { return ((k >> 4) & 1) * 8; }
-// fp16 B tiles (8 halves per 16-byte chunk). [N x K]: a 32-deep row is 4
-// chunks; chunk c of row r sits at c ^ ((r >> 2) & 3), so the 16 rows of a
-// 16-lane slice of ds_read_b128 (row pitch 64 bytes) cover all 64 banks.
-// [K x N]: chunk c of row k sits at c ^ (4 ((k >> 4) & 1)), moving rows k and
-// k + 16 (the two half-waves of a fragment read) 64 bytes apart in the banks.
-__device__ __forceinline__ int swz_rows_h(int r) { return (r >> 2) & 3; }
-__device__ __forceinline__ int swz_kn_h(int k) { return ((k >> 4) & 1) * 4; }
-
-//
-// Workgroup layout: WGM x WGN waves, each owning a (BM / WGM) x (BN / WGN)
-// block of the tile as 32 x 32 MFMA blocks, and S LDS stages per operand.
-// 128 x 128 and smaller tiles: 4 waves, 2 stages (64 KB for 128 x 128 fp32),
-// two workgroups per CU. 256 x 128: 8 waves, 3 stages (144 KB), one
-// workgroup per CU; a stage's loads then have two K tiles of MFMAs to land
-// in, and each byte loaded feeds a third more MFMA work than on 128 x 128.
-template <int BM, int BN>
-struct TileCfg {
-  static constexpr bool kBig = BM == 256;
-  static constexpr int WGM = kBig ? 4 : 2;
-  static constexpr int WGN = 2;
-  static constexpr int kWaves = WGM * WGN;
-  static constexpr int kThreads = 64 * kWaves;
-  static constexpr int S = kBig ? 3 : 2;
-  static constexpr int kMinBlocks = kBig ? 1 : 2;  // workgroups per CU
-  static constexpr int WM = BM / WGM;
-  static constexpr int WN = BN / WGN;
-  static constexpr int MB = WM / 32;
-  static constexpr int NB = WN / 32;
-  static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile");
-};
-
-template <int BM, int BN>
-using TileAcc = floatx16[TileCfg<BM, BN>::MB][TileCfg<BM, BN>::NB];
-
 // The stages of each operand are separate LDS variables and the K loop is
 // unrolled by S, so every LDS access names its buffer statically: the
 // compiler tracks direct loads per variable, and a fragment read of one stage
 // then waits only for that stage's loads, not for the ones in flight into the
 // others.
 //
-// B may also be fp16 (BT = _Float16): its tiles are loaded into LDS as raw
-// halves, half the bytes of an fp32 tile, and converted to fp32 as each lane
-// reads its fragment, so the MFMAs and the accumulation are those of the fp32
-// path (fp16 -> fp32 is exact).
-//
 // EDGE: M and N need not be multiples of the tile. Loads of rows (A, [N x K]
 // B) or 16-byte column chunks ([K x N] B) past the matrix read the last valid
 // one instead -- in bounds, and only ever multiplied into accumulators whose
 // C element is outside the matrix -- and those elements are not stored.
 //
-// The K tiles [kt0, kt1) of the output tile at (m0, n0), accumulated into
-// acc (zeroed here); ends with a barrier, so a following call may refill
-// the LDS stages.
-template <int BM, int BN, bool BNK, typename BT, bool EDGE>
-__device__ __forceinline__ void dma_tile(const float* __restrict__ A, const BT* __restrict__ B,
-                                         int M, int N, int K, int m0, int n0, int kt0, int kt1,
-                                         TileAcc<BM, BN>& acc) {
-  using C = TileCfg<BM, BN>;
-  constexpr bool HB = std::is_same<BT, _Float16>::value;
-  constexpr int BV = 16 / static_cast<int>(sizeof(BT));  // B elements per 16-byte chunk
-  constexpr int S = C::S;
-  constexpr int MB = C::MB;
-  constexpr int NB = C::NB;
-  constexpr int A_CH = BM * BK / 4;  // 16-byte chunks of an A tile
-  constexpr int B_CH = BN * BK / BV;
-  constexpr int A_INST = A_CH / C::kThreads;  // chunk loads per thread (= per wave instruction count)
-  constexpr int B_INST = B_CH / C::kThreads;
-  constexpr int kLoads = A_INST + B_INST;     // direct loads per thread per K tile
-  constexpr int BROW = BN / BV;               // chunks per [K x N] B row
-  static_assert(A_CH % C::kThreads == 0 && B_CH % C::kThreads == 0, "tile shape");
-  static_assert(S == 2 || S == 3, "stages");
-  __shared__ __attribute__((aligned(1024))) float As0[BM * BK];
-  __shared__ __attribute__((aligned(1024))) float As1[BM * BK];
-  __shared__ __attribute__((aligned(1024))) float As2[S > 2 ? BM * BK : 1];
-  __shared__ __attribute__((aligned(1024))) BT Bs0[BN * BK];
-  __shared__ __attribute__((aligned(1024))) BT Bs1[BN * BK];
-  __shared__ __attribute__((aligned(1024))) BT Bs2[S > 2 ? BN * BK : 1];
+// The output tile at (m0, n0), accumulated into acc (zeroed here).
+template <bool BNK, bool EDGE>
+__device__ __forceinline__ void dma_tile(const float* __restrict__ A, const float* __restrict__ B,
+                                         int M, int N, int K, int m0, int n0, floatx16& acc) {
+  constexpr int S = 2;
+  constexpr int INST = f32::INST;
+  constexpr int kLoads = 2 * INST;        // direct loads per thread per K tile
+  constexpr int BROW = f32::BN / 4;       // chunks per [K x N] B row
+  __shared__ __attribute__((aligned(1024))) float As0[f32::BM * BK];
+  __shared__ __attribute__((aligned(1024))) float As1[f32::BM * BK];
+  __shared__ __attribute__((aligned(1024))) float Bs0[f32::BN * BK];
+  __shared__ __attribute__((aligned(1024))) float Bs1[f32::BN * BK];
   auto a_stage = [&](auto st) -> float* {
     if constexpr (decltype(st)::value == 0) return As0;
-    else if constexpr (decltype(st)::value == 1) return As1;
-    else return As2;
+    else return As1;
   };
-  auto b_stage = [&](auto st) -> BT* {
+  auto b_stage = [&](auto st) -> float* {
     if constexpr (decltype(st)::value == 0) return Bs0;
-    else if constexpr (decltype(st)::value == 1) return Bs1;
-    else return Bs2;
+    else return Bs1;
   };
 
   const int t = threadIdx.x;
@@ -432,117 +367,78 @@ __device__ __forceinline__ void dma_tile(const float* __restrict__ A, const BT* 
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int li = lane & 31;
   const int lg = lane >> 5;
-  const int wm = wave / C::WGN;
-  const int wn = wave % C::WGN;
+  const int wm = wave / f32::WGN;
+  const int wn = wave % f32::WGN;
 
   // Direct loads of K tile kt into one stage. Wave w's j-th instruction fills
   // chunk slots (waves j + w) * 64 + lane. Each lane's byte offset from the
   // tile's corner is the same for every K tile (a_off, b_off); only the
   // descriptor's base moves, by BK columns of A and BK rows (or columns) of B.
-  unsigned a_off[A_INST];
-  unsigned b_off[B_INST];
+  unsigned a_off[INST];
+  unsigned b_off[INST];
 #pragma unroll
-  for (int j = 0; j < A_INST; ++j) {
-    const int slot = (C::kWaves * j + wave) * 64 + lane;
+  for (int j = 0; j < INST; ++j) {
+    const int slot = (f32::kWaves * j + wave) * 64 + lane;
     const int r = slot >> 3;
     const int c = (slot & 7) ^ swz_rows(r);
     const int row = EDGE ? min(m0 + r, M - 1) - m0 : r;
     a_off[j] = static_cast<unsigned>(row * K + 4 * c) * 4u;
-  }
-#pragma unroll
-  for (int j = 0; j < B_INST; ++j) {
-    const int slot = (C::kWaves * j + wave) * 64 + lane;
     if constexpr (BNK) {
-      const int r = HB ? slot >> 2 : slot >> 3;
-      const int c = HB ? (slot & 3) ^ swz_rows_h(r) : (slot & 7) ^ swz_rows(r);
-      const int row = EDGE ? min(n0 + r, N - 1) - n0 : r;
-      b_off[j] = static_cast<unsigned>(row * K + BV * c) * static_cast<unsigned>(sizeof(BT));
+      const int rb = EDGE ? min(n0 + r, N - 1) - n0 : r;
+      b_off[j] = static_cast<unsigned>(rb * K + 4 * c) * 4u;
     } else {
       const int k = slot / BROW;
-      const int c = (slot % BROW) ^ (HB ? swz_kn_h(k) : swz_kn(k));
-      // N % BV == 0: a chunk is inside the row or wholly past it.
-      const int col = EDGE ? min(n0 + BV * c, N - BV) - n0 : BV * c;
-      b_off[j] = static_cast<unsigned>(k * N + col) * static_cast<unsigned>(sizeof(BT));
+      const int cb = (slot % BROW) ^ swz_kn(k);
+      // N % 4 == 0: a chunk is inside the row or wholly past it.
+      const int col = EDGE ? min(n0 + 4 * cb, N - 4) - n0 : 4 * cb;
+      b_off[j] = static_cast<unsigned>(k * N + col) * 4u;
     }
   }
   const long long a_len = static_cast<long long>(M) * K;
   const long long b_len = static_cast<long long>(N) * K;
-  auto fetch = [&](float* as, BT* bs, int kt) {
+  auto fetch = [&](float* as, float* bs, int kt) {
     const int k0 = kt * BK;
     const long long a0 = static_cast<long long>(m0) * K + k0;
     const long long b0 = BNK ? static_cast<long long>(n0) * K + k0 : static_cast<long long>(k0) * N + n0;
     const unsigned a_bytes = bytes_left<float>(a_len, a0);
-    const unsigned b_bytes = bytes_left<BT>(b_len, b0);
+    const unsigned b_bytes = bytes_left<float>(b_len, b0);
 #pragma unroll
-    for (int j = 0; j < A_INST; ++j)
-      lds_buf16(A + a0, a_bytes, a_off[j], as + 4 * (C::kWaves * j + wave) * 64);
+    for (int j = 0; j < INST; ++j)
+      lds_buf16(A + a0, a_bytes, a_off[j], as + 4 * (f32::kWaves * j + wave) * 64);
 #pragma unroll
-    for (int j = 0; j < B_INST; ++j)
-      lds_buf16(B + b0, b_bytes, b_off[j], bs + BV * (C::kWaves * j + wave) * 64);
+    for (int j = 0; j < INST; ++j)
+      lds_buf16(B + b0, b_bytes, b_off[j], bs + 4 * (f32::kWaves * j + wave) * 64);
   };
 
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mb][nb][v] = 0.0f;
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
 
   // Fragments of one quarter of a K tile (MFMA k-slices s = 4 q .. 4 q + 3):
   // lane (li, lg) holds A[row][16 lg + s] and B[16 lg + s][col].
   struct Quarter {
-    floatx4 a[MB];
-    float b[NB][4];
+    floatx4 a;
+    float b[4];
   };
-  auto read_q = [&](const float* as, const BT* bs, int q, Quarter& f) {
+  auto read_q = [&](const float* as, const float* bs, int q, Quarter& f) {
+    const int r = wm * 32 + li;
+    f.a = *reinterpret_cast<const floatx4*>(as + 4 * (r * 8 + ((lg * 4 + q) ^ swz_rows(r))));
+    const int n = wn * 32 + li;
+    if constexpr (BNK) {
+      const floatx4 v = *reinterpret_cast<const floatx4*>(bs + 4 * (n * 8 + ((lg * 4 + q) ^ swz_rows(n))));
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int r = wm * C::WM + mb * 32 + li;
-      const int c = (lg * 4 + q) ^ swz_rows(r);
-      f.a[mb] = *reinterpret_cast<const floatx4*>(as + 4 * (r * 8 + c));
-    }
+      for (int e = 0; e < 4; ++e) f.b[e] = v[e];
+    } else {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      if constexpr (BNK && !HB) {
-        const int r = wn * C::WN + nb * 32 + li;
-        const int c = (lg * 4 + q) ^ swz_rows(r);
-        const floatx4 v = *reinterpret_cast<const floatx4*>(bs + 4 * (r * 8 + c));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f.b[nb][e] = v[e];
-      } else if constexpr (BNK) {
-        // Row r holds k = 0..31 as 4 chunks of 8; this lane's k = 16 lg + 4 q + e
-        // are halves 4 (q & 1) .. 4 (q & 1) + 3 of chunk 2 lg + q / 2.
-        const int r = wn * C::WN + nb * 32 + li;
-        const int c = (lg * 2 + (q >> 1)) ^ swz_rows_h(r);
-        const _Float16* p = bs + 8 * (r * 4 + c) + 4 * (q & 1);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f.b[nb][e] = static_cast<float>(p[e]);
-      } else {
-        const int n = wn * C::WN + nb * 32 + li;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int k = lg * 16 + 4 * q + e;
-          if constexpr (HB) {
-            const int c = (n >> 3) ^ swz_kn_h(k);
-            f.b[nb][e] = static_cast<float>(bs[8 * (k * BROW + c) + (n & 7)]);
-          } else {
-            const int c = (n >> 2) ^ swz_kn(k);
-            f.b[nb][e] = bs[4 * (k * BROW + c) + (n & 3)];
-          }
-        }
+      for (int e = 0; e < 4; ++e) {
+        const int k = lg * 16 + 4 * q + e;
+        f.b[e] = bs[4 * (k * BROW + ((n >> 2) ^ swz_kn(k))) + (n & 3)];
       }
     }
   };
   auto mma_q = [&](const Quarter& f) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[mb][e], f.b[nb][e], acc[mb][nb], 0, 0, 0);
-      }
-    }
+    for (int e = 0; e < 4; ++e)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[e], f.b[e], acc, 0, 0, 0);
   };
 
   // Software pipeline over quarters: each quarter's fragments are read while
@@ -553,7 +449,7 @@ __device__ __forceinline__ void dma_tile(const float* __restrict__ A, const BT* 
   // ends every wave's reads of the current stage, which the fetch after it
   // refills with the tile S steps ahead. That fetch and the read after the
   // barrier are unconditional so that nothing splits the block: near the end
-  // the fetch loads tile kt1 - 1 again into a finished stage and the read
+  // the fetch loads the last tile again into a finished stage and the read
   // takes a stale quarter that is never used. Scheduling barriers keep each
   // quarter's reads ahead of the previous quarter's MFMAs.
   auto pin = [] {
@@ -563,11 +459,10 @@ __device__ __forceinline__ void dma_tile(const float* __restrict__ A, const BT* 
     __builtin_amdgcn_sched_barrier(0);
 #endif
   };
-  // After the stage barrier every wave of the workgroup resumes at once (the
-  // two on each SIMD, on 256 x 128 tiles): two MFMAs go first, then each of
-  // the fetch's loads, with its address arithmetic, behind one more MFMA, so
-  // the matrix core stays busy while they issue (4096^3: 947 us with the
-  // loads first, 921 us interleaved).
+  // After the stage barrier every wave of the workgroup resumes at once: two
+  // MFMAs go first, then each of the fetch's loads, with its address
+  // arithmetic, behind one more MFMA, so the matrix core stays busy while they
+  // issue.
   auto pin_after_barrier = [] {
 #if defined(__HIP_DEVICE_COMPILE__)
     __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // MFMAs
@@ -581,12 +476,13 @@ __device__ __forceinline__ void dma_tile(const float* __restrict__ A, const BT* 
     __builtin_amdgcn_sched_barrier(0);
 #endif
   };
+  const int nk = K / BK;
   Quarter x, y;
   auto tile = [&](auto st, int kt) {
     constexpr int cur = decltype(st)::value;
     using Next = std::integral_constant<int, (cur + 1) % S>;
     const float* as = a_stage(st);
-    const BT* bs = b_stage(st);
+    const float* bs = b_stage(st);
     read_q(as, bs, 1, y);
     mma_q(x);
     pin();
@@ -597,298 +493,92 @@ __device__ __forceinline__ void dma_tile(const float* __restrict__ A, const BT* 
     mma_q(x);
     pin();
     stage_barrier<(S - 2) * kLoads>();
-    fetch(a_stage(st), b_stage(st), min(kt + S, kt1 - 1));
+    fetch(a_stage(st), b_stage(st), min(kt + S, nk - 1));
     read_q(a_stage(Next{}), b_stage(Next{}), 0, x);
     mma_q(y);
     pin_after_barrier();
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
 
-  fetch(As0, Bs0, kt0);
-  fetch(As1, Bs1, min(kt0 + 1, kt1 - 1));
-  if constexpr (S > 2) fetch(As2, Bs2, min(kt0 + 2, kt1 - 1));
+  fetch(As0, Bs0, 0);
+  fetch(As1, Bs1, min(1, nk - 1));
   stage_barrier<(S - 1) * kLoads>();
   read_q(As0, Bs0, 0, x);
-  int kt = kt0;
-  for (; kt + S - 1 < kt1; kt += S) {
+  int kt = 0;
+  for (; kt + 1 < nk; kt += S) {
     tile(I0{}, kt);
     tile(I1{}, kt + 1);
-    if constexpr (S > 2) tile(I2{}, kt + 2);
   }
-  if (kt < kt1) tile(I0{}, kt);
-  if constexpr (S > 2) {
-    if (kt + 1 < kt1) tile(I1{}, kt + 1);
-  }
+  if (kt < nk) tile(I0{}, kt);
   wait_all_memory();
   __syncthreads();
 }
 
-// Stores a tile's accumulators: element (r, c) of the tile to out[r * ld + c]
-// (out at the tile's first element), rows < rows_left and columns < cols_left
-// only (EDGE).
-template <int BM, int BN, bool EDGE>
-__device__ __forceinline__ void store_acc(const TileAcc<BM, BN>& acc, float* __restrict__ out,
-                                          long long ld, int rows_left, int cols_left) {
-  using C = TileCfg<BM, BN>;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int li = lane & 31;
-  const int lg = lane >> 5;
-  const int wm = wave / C::WGN;
-  const int wn = wave % C::WGN;
-#if defined(__HIP_DEVICE_COMPILE__)
-  // In the stream-K kernel's tile loop the per-element offsets row ld + col
-  // are loop-invariant; hoisted they held registers through the K loop (36
-  // bytes of spills at 128 x 128). An opaque ld keeps them here.
-  asm volatile("" : "+s"(ld));
-#endif
-#pragma unroll
-  for (int mb = 0; mb < C::MB; ++mb) {
-#pragma unroll
-    for (int nb = 0; nb < C::NB; ++nb) {
-      const int col = wn * C::WN + nb * 32 + li;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = wm * C::WM + mb * 32 + 8 * (v >> 2) + 4 * lg + (v & 3);
-        if (!EDGE || (row < rows_left && col < cols_left)) out[row * ld + col] = acc[mb][nb][v];
-      }
-    }
-  }
-}
-
-template <int BM, int BN, bool BNK, typename BT = float, bool EDGE = false>
-__global__ __launch_bounds__((TileCfg<BM, BN>::kThreads), (TileCfg<BM, BN>::kMinBlocks)) void
-gemm_f32_mfma_dma_kernel(const float* __restrict__ A, const BT* __restrict__ B,
-                         float* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n) {
+template <bool BNK, bool EDGE>
+__global__ __launch_bounds__(f32::kThreads, 2) void gemm_f32_mfma_dma_kernel(
+    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N,
+    int K, int tiles_m, int tiles_n) {
   int tm, tn;
   tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM;
-  const int n0 = tn * BN;
-  TileAcc<BM, BN> acc;
-  dma_tile<BM, BN, BNK, BT, EDGE>(A, B, M, N, K, m0, n0, 0, K / BK, acc);
-  store_acc<BM, BN, EDGE>(acc, C + static_cast<long long>(m0) * N + n0, N, M - m0, N - n0);
-}
-
-// Stream-K tail (full tiles only): T tiles, of which the first `dp` in
-// tile_of order are computed whole by workgroups 0 .. dp - 1 (one round of
-// one per CU), and the remaining T - dp tiles' k-iterations are split evenly
-// over the workgroups dp .. dp + nsk - 1 (nsk = min(dp, I): none is empty):
-// workgroup dp + s takes iterations [s I / nsk, (s + 1) I / nsk) of the
-// tail's I = (T - dp) nk, tile by tile.
-// Running beside the data-parallel round (two workgroups per CU), every CU
-// then does the same work whatever T is (512 x 11008 x 4096: 344 tiles on
-// 256 CUs). A tail tile one workgroup covers whole is stored to C; a split
-// tile leaves one record per workgroup (slot 0 its first tile, slot 1 its
-// last), which gemm_sk_fixup_kernel adds in workgroup order.
-struct SkPlan {
-  int dp = 0;        // data-parallel tiles (one per CU)
-  int nsk = 0;       // stream-K workgroups
-  int nk = 0;        // K tiles per output tile
-  long long I = 0;   // tail iterations (tail tiles x nk)
-};
-
-__host__ __device__ inline long long sk_begin(long long s, const SkPlan& p) {
-  return s * p.I / p.nsk;
-}
-
-// Stream-K workgroup whose range holds tail iteration it.
-__device__ inline long long sk_worker(long long it, const SkPlan& p) {
-  long long s = (it * p.nsk + p.nsk - 1) / p.I;
-  if (s >= p.nsk) s = p.nsk - 1;
-  while (s + 1 < p.nsk && sk_begin(s + 1, p) <= it) ++s;
-  while (s > 0 && sk_begin(s, p) > it) --s;
-  return s;
-}
-
-template <int BM, int BN, bool BNK, typename BT>
-__global__ __launch_bounds__(kThreads, 2) void gemm_sk_kernel(
-    const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ C,
-    float* __restrict__ rec, int M, int N, int K, int tiles_m, int tiles_n, SkPlan plan) {
-  TileAcc<BM, BN> acc;
-  // One loop for both kinds of workgroup (a single inlined copy of the tile
-  // loop): a data-parallel workgroup g covers iterations [0, nk) of tile g; a
-  // stream-K workgroup its share of the tail, whose tile t is tile dp + t.
-  const int g = blockIdx.x;
-  const bool dp = g < plan.dp;
-  const long long s = dp ? 0 : g - plan.dp;
-  const long long i0 = dp ? 0 : sk_begin(s, plan);
-  const long long i1 = dp ? plan.nk : sk_begin(s + 1, plan);
-  const int first_tile = dp ? g : plan.dp;
-  for (long long it = i0; it < i1;) {
-    const long long t = it / plan.nk;
-    const int ka = static_cast<int>(it - t * plan.nk);
-    const long long tend = (t + 1) * plan.nk;
-    const int kb = static_cast<int>((i1 < tend ? i1 : tend) - t * plan.nk);
-    int tm, tn;
-    tile_of(first_tile + static_cast<int>(t), tiles_m, tiles_n, tm, tn);
-    const int m0 = tm * BM;
-    const int n0 = tn * BN;
-    dma_tile<BM, BN, BNK, BT, false>(A, B, M, N, K, m0, n0, ka, kb, acc);
-    if (ka == 0 && kb == plan.nk) {
-      store_acc<BM, BN, false>(acc, C + static_cast<long long>(m0) * N + n0, N, BM, BN);
-    } else {
-      const int slot = it == i0 ? 0 : 1;
-      store_acc<BM, BN, false>(acc, rec + (s * 2 + slot) * static_cast<long long>(BM * BN), BN,
-                               BM, BN);
-    }
-    it = t * plan.nk + kb;
-  }
-}
-
-// Split tail tiles: C = the tile's records added in workgroup order. One
-// block per (tail tile, 1024 elements); tiles one workgroup covered whole are
-// skipped (already stored).
-template <int BM, int BN, bool EDGE = false>
-__global__ __launch_bounds__(256) void gemm_sk_fixup_kernel(const float* __restrict__ rec,
-                                                            float* __restrict__ C, int M, int N,
-                                                            int tiles_m, int tiles_n,
-                                                            SkPlan plan) {
-  const long long t = blockIdx.x;
-  const long long sf = sk_worker(t * plan.nk, plan);
-  const long long sl = sk_worker(t * plan.nk + plan.nk - 1, plan);
-  if (sf == sl) return;
-  // workgroups after sf start inside the tile (slot 0); sf only when it
-  // starts exactly at the tile
-  const int slot_f = sk_begin(sf, plan) == t * plan.nk ? 0 : 1;
-  const int e = 4 * (static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x));
-  floatx4 v = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  // (unrolled so a group's loads are in flight together; the adds keep
-  // workgroup order)
-#pragma unroll 8
-  for (long long s = sf; s <= sl; ++s) {
-    const long long r = s * 2 + (s == sf ? slot_f : 0);
-    v += *reinterpret_cast<const floatx4*>(rec + r * static_cast<long long>(BM * BN) + e);
-  }
-  int tm, tn;
-  tile_of(plan.dp + static_cast<int>(t), tiles_m, tiles_n, tm, tn);
-  const int row = tm * BM + e / BN;
-  const int col = tn * BN + e % BN;
-  float* dst = C + static_cast<long long>(row) * N + col;
-  if constexpr (!EDGE) {
-    *reinterpret_cast<floatx4*>(dst) = v;
-  } else if (row < M) {
+  const int m0 = tm * f32::BM;
+  const int n0 = tn * f32::BN;
+  floatx16 acc;
+  dma_tile<BNK, EDGE>(A, B, M, N, K, m0, n0, acc);
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int col = n0 + (wave % f32::WGN) * 32 + (lane & 31);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (col + q < N) dst[q] = v[q];
+  for (int v = 0; v < 16; ++v) {
+    const int row = m0 + (wave / f32::WGN) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+    if (!EDGE || (row < M && col < N)) C[static_cast<long long>(row) * N + col] = acc[v];
   }
-}
-
-// The direct-load kernel can be switched off (ENGINE_GEMM_NO_DMA=1) to
-// compare it with the register-staged kernel on the same shapes.
-bool dma_enabled() {
-  static const bool on = [] {
-    const char* v = std::getenv("ENGINE_GEMM_NO_DMA");
-    return !(v != nullptr && v[0] == '1');
-  }();
-  return on;
 }
 
 // Direct loads need K % BK == 0, 16-byte aligned operands and 16-byte
 // aligned B rows ([K x N] rows of N elements; [N x K] rows of K), and every
-// lane's byte offset from a tile's corner (up to BM rows of A, BN rows of an
+// lane's byte offset from a tile's corner (up to 64 rows of A, 64 rows of an
 // [N x K] B or BK rows of a [K x N] B) must fit the 31 bits of a buffer
 // load's offset.
-template <int BM, int BN, typename BT, bool BNK>
+template <bool BNK>
 bool direct_ok(const GemmArgs& a) {
-  constexpr long long kBVec = 16 / static_cast<long long>(sizeof(BT));
   constexpr long long kLim = 0x7fffffffLL;
-  const long long b_span = BNK ? static_cast<long long>(BN) * a.K : static_cast<long long>(BK) * a.N;
-  return dma_enabled() && a.K % BK == 0 && aligned_to(a.A, 16) && aligned_to(a.B, 16) &&
-         (BNK || a.N % kBVec == 0) && static_cast<long long>(BM) * a.K * 4 <= kLim &&
-         b_span * static_cast<long long>(sizeof(BT)) <= kLim;
+  const long long b_span = BNK ? static_cast<long long>(f32::BN) * a.K : static_cast<long long>(BK) * a.N;
+  return a.b == Elem::F32 && a.K % BK == 0 && aligned_to(a.A, 16) && aligned_to(a.B, 16) &&
+         (BNK || a.N % 4 == 0) && static_cast<long long>(f32::BM) * a.K * 4 <= kLim &&
+         b_span * 4 <= kLim;
 }
 
-// The 256 x 128 tile can be switched off (ENGINE_GEMM_NO_BIG=1) to compare
-// it with 128 x 128 on the same shapes.
-bool big_tile_enabled() {
-  static const bool on = [] {
-    const char* v = std::getenv("ENGINE_GEMM_NO_BIG");
-    return !(v != nullptr && v[0] == '1');
-  }();
-  return on;
+// Estimated time of the 64 x 64 FP32 tiles: per K tile 0.48 us with one
+// workgroup on a CU (1024^3: 256 tiles, 17.9 us) and 0.94 us for a pair (512 x
+// 4096 x 4096: 512 tiles, 120 us).
+double f32_us(const GemmArgs& a, long long cus) {
+  const long long tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
+  const double nk = static_cast<double>(a.K / BK);
+  return tiles <= cus ? 0.48 * nk : 0.94 * nk * static_cast<double>((tiles + 2 * cus - 1) / (2 * cus));
 }
 
-template <int BM, int BN, typename BT, bool BNK>
-void run_gemm(const GemmArgs& a, hipStream_t stream) {
-  constexpr int kBVec = 16 / static_cast<int>(sizeof(BT));
-  const bool va = (a.K % 4 == 0) && aligned_to(a.A, 16);
-  // B rows run along N ([K x N]) or along K ([N x K]).
-  const bool vb = ((BNK ? a.K : a.N) % kBVec == 0) && aligned_to(a.B, 16);
+template <bool BNK>
+void run_gemm_f32(const GemmArgs& a, hipStream_t stream) {
   const int M = static_cast<int>(a.M);
   const int N = static_cast<int>(a.N);
   const int K = static_cast<int>(a.K);
-  const int tiles_m = (M + BM - 1) / BM;
-  const int tiles_n = (N + BN - 1) / BN;
+  const int tiles_m = (M + f32::BM - 1) / f32::BM;
+  const int tiles_n = (N + f32::BN - 1) / f32::BN;
   const long long ntiles = static_cast<long long>(tiles_m) * tiles_n;
   ENG_CHECK(ntiles <= 0x7fffffffLL, "matmul: too many tiles for one launch");
   const dim3 grid(static_cast<unsigned>(ntiles));
-  const BT* B = static_cast<const BT*>(a.B);
-  if (direct_ok<BM, BN, BT, BNK>(a)) {
-    // Whole tiles take the plain kernel, ragged M / N its EDGE form.
-    constexpr int kDmaThreads = TileCfg<BM, BN>::kThreads;
-    if (M % BM == 0 && N % BN == 0) {
-      gemm_f32_mfma_dma_kernel<BM, BN, BNK, BT, false><<<grid, kDmaThreads, 0, stream>>>(
-          a.A, B, a.C, M, N, K, tiles_m, tiles_n);
-    } else {
-      gemm_f32_mfma_dma_kernel<BM, BN, BNK, BT, true><<<grid, kDmaThreads, 0, stream>>>(
-          a.A, B, a.C, M, N, K, tiles_m, tiles_n);
-    }
-    ENG_LAUNCH_CHECK();
-    return;
-  }
-  if constexpr (TileCfg<BM, BN>::kBig) {
-    // big_tile() only picks 256 x 128 when the direct loads apply
-    ENG_CHECK(false, "matmul: 256-row tiles need the direct-load kernel");
-  } else {
-#define ENG_GEMM_LAUNCH(VA_, VB_)                                                    \
-    gemm_f32_mfma_kernel<BM, BN, BT, BNK, VA_, VB_><<<grid, kThreads, 0, stream>>>( \
-        a.A, B, a.C, M, N, K, tiles_m, tiles_n)
-    if (va && vb) {
-      ENG_GEMM_LAUNCH(true, true);
-    } else if (va) {
-      ENG_GEMM_LAUNCH(true, false);
-    } else if (vb) {
-      ENG_GEMM_LAUNCH(false, true);
-    } else {
-      ENG_GEMM_LAUNCH(false, false);
-    }
-#undef ENG_GEMM_LAUNCH
-    ENG_LAUNCH_CHECK();
-  }
+  const float* B = static_cast<const float*>(a.B);
+  // Whole tiles take the plain kernel, ragged M / N its EDGE form.
+  if (M % f32::BM == 0 && N % f32::BN == 0)
+    gemm_f32_mfma_dma_kernel<BNK, false><<<grid, f32::kThreads, 0, stream>>>(a.A, B, a.C, M, N, K,
+                                                                            tiles_m, tiles_n);
+  else
+    gemm_f32_mfma_dma_kernel<BNK, true><<<grid, f32::kThreads, 0, stream>>>(a.A, B, a.C, M, N, K,
+                                                                           tiles_m, tiles_n);
+  ENG_LAUNCH_CHECK();
 }
 
-// Tile shape: the largest of 128 x 128, 128 x 64, 64 x 64 whose makespan (rounds
-// of one tile per CU, times the tile's share of the work) is not worse than a
-// smaller shape's. Smaller tiles re-read A and B more, so ties go to the larger
-// -- except that 64 x 64 wins a tie with 128 x 64 when 128 x 64 leaves at most
-// one workgroup per CU: two co-resident 64 x 64 workgroups hide each other's
-// latency (MI355X: 512 x 4096 x 11008 361 vs 376 us, 512 x 4096 x 4096 138 vs
-// 142 us). The same preference measured slower one step up (1024 x 4096 x 4096:
-// 256 tiles of 128 x 128 258 us, 512 of 128 x 64 272 us) and with more than one
-// workgroup per CU (512 x 11008 x 4096: 128 x 64 411 us, 64 x 64 420 us).
-enum class Tile { T128x128, T128x64, T64x64 };
-
-Tile choose_tile(long long M, long long N) {
-  const long long cus = device_cu_count();
-  auto tiles = [&](long long bm, long long bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  auto makespan = [&](long long bm, long long bn) {
-    const long long rounds = (tiles(bm, bn) + cus - 1) / cus;
-    return static_cast<double>(rounds) * static_cast<double>(bm * bn) / (128.0 * 128.0);
-  };
-  const double t1 = makespan(128, 128);
-  const double t2 = makespan(128, 64);
-  const double t3 = makespan(64, 64);
-  if (t1 <= t2 && t1 <= t3) return Tile::T128x128;
-  if (t2 < t3 || (t2 == t3 && tiles(128, 64) > cus)) return Tile::T128x64;
-  return Tile::T64x64;
-}
-
-// Stream-K tail for 128 x 128 tiles when their count T falls between one
-// and two rounds of one tile per CU (CUs < T < 2 CUs; every other shape
-// keeps choose_tile's tiling): full tiles and the direct-load conditions
-// only. ENGINE_GEMM_NO_SK=1 switches it off.
 // The single-launch small-GEMM kernel can be switched off
 // (ENGINE_GEMM_NO_SMALL=1).
 bool small_enabled() {
@@ -905,34 +595,6 @@ bool sk_enabled() {
     return !(v != nullptr && v[0] == '1');
   }();
   return on;
-}
-
-template <typename BT, bool BNK>
-bool run_gemm_sk(const GemmArgs& a, hipStream_t stream) {
-  constexpr int BM = 128, BN = 128;
-  if (!sk_enabled() || !direct_ok<BM, BN, BT, BNK>(a)) return false;
-  if (a.M % BM != 0 || a.N % BN != 0 || a.K / BK < 8) return false;
-  const long long cus = device_cu_count();
-  const int tiles_m = static_cast<int>(a.M / BM);
-  const int tiles_n = static_cast<int>(a.N / BN);
-  const long long T = static_cast<long long>(tiles_m) * tiles_n;
-  if (T <= cus || T >= 2 * cus) return false;
-  SkPlan plan;
-  plan.dp = static_cast<int>(cus);
-  plan.nk = static_cast<int>(a.K / BK);
-  plan.I = (T - cus) * plan.nk;
-  plan.nsk = static_cast<int>(std::min<long long>(plan.dp, plan.I));
-  StreamScratch records(stream, static_cast<std::size_t>(plan.nsk) * 2 * BM * BN * sizeof(float), 2);
-  float* rec = static_cast<float*>(records.get());
-  const BT* B = static_cast<const BT*>(a.B);
-  const int M = static_cast<int>(a.M), N = static_cast<int>(a.N), K = static_cast<int>(a.K);
-  gemm_sk_kernel<BM, BN, BNK, BT><<<static_cast<unsigned>(plan.dp + plan.nsk), kThreads, 0, stream>>>(
-      a.A, B, a.C, rec, M, N, K, tiles_m, tiles_n, plan);
-  ENG_LAUNCH_CHECK();
-  gemm_sk_fixup_kernel<BM, BN><<<dim3(static_cast<unsigned>(T - cus), BM * BN / 1024), 256, 0,
-                                 stream>>>(rec, a.C, M, N, tiles_m, tiles_n, plan);
-  ENG_LAUNCH_CHECK();
-  return true;
 }
 
 // Small GEMMs in one launch: one 32 x 32 tile of C per workgroup, its four
@@ -1005,60 +667,63 @@ __global__ __launch_bounds__(256) void gemm_small_splitk_kernel(const float* __r
   }
 }
 
-template <typename BT, bool BNK>
-bool run_gemm_small(const GemmArgs& a, hipStream_t stream) {
-  if constexpr (BNK || !std::is_same<BT, float>::value) {
-    return false;
-  } else {
-    if (!small_enabled() || a.M % 32 != 0 || a.N % 32 != 0 || a.K % 256 != 0 ||
-        !aligned_to(a.A, 16))
-      return false;
-    const long long cus = device_cu_count();
-    if (2 * (a.M / 64) * (a.N / 64) > cus) return false;  // 64 x 64 tiles fill half the CUs
-    const long long tiles = (a.M / 32) * (a.N / 32);
-    ENG_CHECK(tiles <= 0x7fffffffLL, "matmul: too many tiles for one launch");
-    gemm_small_splitk_kernel<<<static_cast<unsigned>(tiles), 256, 0, stream>>>(
-        a.A, static_cast<const float*>(a.B), a.C, static_cast<int>(a.M), static_cast<int>(a.N),
-        static_cast<int>(a.K), static_cast<int>(a.N / 32));
-    ENG_LAUNCH_CHECK();
-    return true;
-  }
+// 16-byte loads of A and B in the register-staged kernel.
+bool staged_vec(const GemmArgs& a) {
+  const long long vb = a.b == Elem::F32 ? 4 : 8;
+  return a.K % 4 == 0 && aligned_to(a.A, 16) && (a.b_nk ? a.K : a.N) % vb == 0 &&
+         aligned_to(a.B, 16);
 }
 
-// 256 x 128 tiles where choose_tile's model takes 128 x 128 and gives the
-// larger tile no longer a makespan (rounds of one tile per CU, times the
-// tile's area: 4096^3 has 512 such tiles against 1024, two rounds of twice
-// the work against four), and the direct loads apply.
-template <typename BT, bool BNK>
-bool big_tile(const GemmArgs& a) {
-  if (!big_tile_enabled() || !direct_ok<256, 128, BT, BNK>(a)) return false;
-  if (choose_tile(a.M, a.N) != Tile::T128x128) return false;
-  const long long cus = device_cu_count();
-  auto rounds = [&](long long bm, long long bn) {
-    return (((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) + cus - 1) / cus;
-  };
-  return 2 * rounds(256, 128) <= rounds(128, 128);
+// Estimated time of the register-staged kernel: per K tile 0.8 us with one
+// workgroup on a CU and 1.05 us for a pair (1000 x 3000 x 200: 17.5 us), more
+// with element loads (200 x 3001 x 64: 4.8 us; 509 x 2051 x 1023: 64.6 us).
+double staged_us(const GemmArgs& a, long long cus) {
+  const long long tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
+  const double nk = static_cast<double>((a.K + BK - 1) / BK);
+  const bool vec = staged_vec(a);
+  if (tiles <= cus) return nk * (vec ? 0.8 : a.b == Elem::F32 ? 1.15 : 1.6);
+  return nk * (vec ? 1.05 : 1.9) * static_cast<double>((tiles + 2 * cus - 1) / (2 * cus));
 }
 
 template <typename BT, bool BNK>
-void run_gemm_tiled(const GemmArgs& a, hipStream_t stream) {
-  if (run_gemm_sk<BT, BNK>(a, stream)) return;
-  if (run_gemm_small<BT, BNK>(a, stream)) return;
-  if (big_tile<BT, BNK>(a)) {
-    run_gemm<256, 128, BT, BNK>(a, stream);
-    return;
-  }
-  switch (choose_tile(a.M, a.N)) {
-    case Tile::T128x128:
-      run_gemm<128, 128, BT, BNK>(a, stream);
-      break;
-    case Tile::T128x64:
-      run_gemm<128, 64, BT, BNK>(a, stream);
-      break;
-    case Tile::T64x64:
-      run_gemm<64, 64, BT, BNK>(a, stream);
-      break;
-  }
+void run_gemm_staged(const GemmArgs& a, hipStream_t stream) {
+  const int M = static_cast<int>(a.M);
+  const int N = static_cast<int>(a.N);
+  const int K = static_cast<int>(a.K);
+  const int tiles_m = (M + f32::BM - 1) / f32::BM;
+  const int tiles_n = (N + f32::BN - 1) / f32::BN;
+  const long long ntiles = static_cast<long long>(tiles_m) * tiles_n;
+  ENG_CHECK(ntiles <= 0x7fffffffLL, "matmul: too many tiles for one launch");
+  const dim3 grid(static_cast<unsigned>(ntiles));
+  const BT* B = static_cast<const BT*>(a.B);
+  if (staged_vec(a))
+    gemm_f32_mfma_kernel<BT, BNK, true, true><<<grid, f32::kThreads, 0, stream>>>(
+        a.A, B, a.C, M, N, K, tiles_m, tiles_n);
+  else
+    gemm_f32_mfma_kernel<BT, BNK, false, false><<<grid, f32::kThreads, 0, stream>>>(
+        a.A, B, a.C, M, N, K, tiles_m, tiles_n);
+  ENG_LAUNCH_CHECK();
+}
+
+bool small_ok(const GemmArgs& a) {
+  return small_enabled() && a.b == Elem::F32 && !a.b_nk && a.M % 32 == 0 && a.N % 32 == 0 &&
+         a.K % 256 == 0 && aligned_to(a.A, 16);
+}
+
+// Estimated time: 0.0065 us per k and round of one 32 x 32 tile per CU (512^3:
+// 5.6 us with about 2.5 of launch; 128 x 4096 x 4096: 63.7 us, two rounds).
+double small_us(const GemmArgs& a, long long cus) {
+  const long long tiles = (a.M / 32) * (a.N / 32);
+  return 0.0065 * static_cast<double>(a.K) * static_cast<double>((tiles + cus - 1) / cus);
+}
+
+void run_gemm_small(const GemmArgs& a, hipStream_t stream) {
+  const long long tiles = (a.M / 32) * (a.N / 32);
+  ENG_CHECK(tiles <= 0x7fffffffLL, "matmul: too many tiles for one launch");
+  gemm_small_splitk_kernel<<<static_cast<unsigned>(tiles), 256, 0, stream>>>(
+      a.A, static_cast<const float*>(a.B), a.C, static_cast<int>(a.M), static_cast<int>(a.N),
+      static_cast<int>(a.K), static_cast<int>(a.N / 32));
+  ENG_LAUNCH_CHECK();
 }
 
 // ---------------------------------------------------------------------------
@@ -1089,7 +754,7 @@ void run_gemm_tiled(const GemmArgs& a, hipStream_t stream) {
 // k rows. Direct loads, the slice read-ahead, the stage hand-over and the
 // interleaved fetch follow the FP32 kernel. Past one round of tiles a last
 // round at most half full, and below half a round every tile, is split by K
-// (gemm_h3_sk_kernel, the plan of gemm_sk_kernel).
+// (gemm_h3_sk_kernel).
 namespace h3 {
 // Tiles of BMT x BNT: 128 x 128 and 128 x 256 on 8 waves, 64 x 128 on 4 waves
 // (two workgroups per CU). BNT / 64 waves along N and the rest along M, each
@@ -1433,7 +1098,7 @@ __global__ __launch_bounds__(4 * BMT, BMT == 64 ? 2 : 1) void gemm_h3_kernel(
                       N - n0);
 }
 
-// Stream-K form (the plan of gemm_sk_kernel): workgroups 0 .. dp - 1 compute
+// Stream-K form: workgroups 0 .. dp - 1 compute
 // tiles 0 .. dp - 1 whole (whole rounds of one tile per resident workgroup,
 // two per CU for 64-row tiles), and the rest split the remaining tiles' K
 // tiles evenly, at most one workgroup per CU after its
@@ -1618,18 +1283,22 @@ void launch_gemm_h3(const GemmH3Args& a, hipStream_t stream) {
 void launch_gemm(const GemmArgs& a, hipStream_t stream) {
   ENG_CHECK(a.M <= 0x7fffffffLL && a.N <= 0x7fffffffLL && a.K <= 0x7fffffffLL,
             "matmul: dimensions must fit in 31 bits");
-  if (a.b == Elem::F32) {
-    if (a.b_nk) {
-      run_gemm_tiled<float, true>(a, stream);
-    } else {
-      run_gemm_tiled<float, false>(a, stream);
-    }
+  // Each kernel's estimate of the call; the smallest runs.
+  const long long cus = device_cu_count();
+  const double never = std::numeric_limits<double>::infinity();
+  const bool direct = a.b_nk ? direct_ok<true>(a) : direct_ok<false>(a);
+  const double small = small_ok(a) ? small_us(a, cus) : never;
+  const double f32 = direct ? f32_us(a, cus) : staged_us(a, cus);
+  if (launch_gemm_split(a, std::min(small, f32), cus, stream)) return;
+  if (small <= f32) {
+    run_gemm_small(a, stream);
+  } else if (direct) {
+    a.b_nk ? run_gemm_f32<true>(a, stream) : run_gemm_f32<false>(a, stream);
+  } else if (a.b == Elem::F32) {
+    a.b_nk ? run_gemm_staged<float, true>(a, stream) : run_gemm_staged<float, false>(a, stream);
   } else {
-    if (a.b_nk) {
-      run_gemm_tiled<_Float16, true>(a, stream);
-    } else {
-      run_gemm_tiled<_Float16, false>(a, stream);
-    }
+    a.b_nk ? run_gemm_staged<_Float16, true>(a, stream)
+           : run_gemm_staged<_Float16, false>(a, stream);
   }
 }
 

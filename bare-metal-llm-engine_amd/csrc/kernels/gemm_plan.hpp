@@ -1,0 +1,109 @@
+// gemm_plan.hpp -- tile numbering and the stream-K plan shared by the GEMM kernels.
+#pragma once
+
+#include "../engine_internal.hpp"
+
+namespace eng {
+namespace {
+
+constexpr int kGroupM = 8;  // tile-rows per raster group
+constexpr int kXcds = 8;
+
+// Workgroup id -> (tile_m, tile_n). Workgroups are handed to XCDs round-robin,
+// so id w runs on XCD w % 8; renumber so XCD x gets a contiguous logical range,
+// then raster that range in groups of kGroupM tile-rows.
+__device__ __forceinline__ void tile_of(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int ntiles = tiles_m * tiles_n;
+  const int q = ntiles / kXcds;
+  const int r = ntiles % kXcds;
+  const int xcd = wg % kXcds;
+  const int local = wg / kXcds;
+  const int logical = xcd * q + (xcd < r ? xcd : r) + local;
+  const int group_size = kGroupM * tiles_n;
+  const int group = logical / group_size;
+  const int first_m = group * kGroupM;
+  const int gm = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
+  const int in_group = logical - group * group_size;
+  tm = first_m + in_group % gm;
+  tn = in_group / gm;
+}
+
+// Stream-K plan: of T tiles in tile_of order the first `dp` are computed whole
+// by workgroups 0 .. dp - 1, and the remaining T - dp tiles' K iterations are
+// split evenly over workgroups dp .. dp + nsk - 1: workgroup dp + s takes
+// iterations [s I / nsk, (s + 1) I / nsk) of the tail's I = (T - dp) nk, tile by
+// tile. A tail tile one workgroup covers whole is stored to C; a split tile
+// leaves one record per workgroup (slot 0 its first tile, slot 1 its last),
+// which gemm_sk_fixup_kernel adds in workgroup order.
+struct SkPlan {
+  int dp = 0;        // data-parallel tiles
+  int nsk = 0;       // stream-K workgroups
+  int nk = 0;        // K tiles per output tile
+  long long I = 0;   // tail iterations (tail tiles x nk)
+};
+
+__host__ __device__ inline long long sk_begin(long long s, const SkPlan& p) {
+  return s * p.I / p.nsk;
+}
+
+// Stream-K workgroup whose range holds tail iteration it.
+__device__ inline long long sk_worker(long long it, const SkPlan& p) {
+  long long s = (it * p.nsk + p.nsk - 1) / p.I;
+  if (s >= p.nsk) s = p.nsk - 1;
+  while (s + 1 < p.nsk && sk_begin(s + 1, p) <= it) ++s;
+  while (s > 0 && sk_begin(s, p) > it) --s;
+  return s;
+}
+
+// Split tail tiles: C = the tile's records added in workgroup order. One
+// block per (tail tile, 1024 elements); tiles one workgroup covered whole are
+// skipped (already stored).
+template <int BM, int BN, bool EDGE = false>
+__global__ __launch_bounds__(256) void gemm_sk_fixup_kernel(const float* __restrict__ rec,
+                                                            float* __restrict__ C, int M, int N,
+                                                            int tiles_m, int tiles_n,
+                                                            SkPlan plan) {
+  typedef float floatx4 __attribute__((ext_vector_type(4)));
+  const long long t = blockIdx.x;
+  const long long sf = sk_worker(t * plan.nk, plan);
+  const long long sl = sk_worker(t * plan.nk + plan.nk - 1, plan);
+  if (sf == sl) return;
+  // workgroups after sf start inside the tile (slot 0); sf only when it
+  // starts exactly at the tile
+  const int slot_f = sk_begin(sf, plan) == t * plan.nk ? 0 : 1;
+  const int e = 4 * (static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x));
+  floatx4 v = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  // (unrolled so a group's loads are in flight together; the adds keep
+  // workgroup order)
+#pragma unroll 8
+  for (long long s = sf; s <= sl; ++s) {
+    const long long r = s * 2 + (s == sf ? slot_f : 0);
+    v += *reinterpret_cast<const floatx4*>(rec + r * static_cast<long long>(BM * BN) + e);
+  }
+  int tm, tn;
+  tile_of(plan.dp + static_cast<int>(t), tiles_m, tiles_n, tm, tn);
+  const int row = tm * BM + e / BN;
+  const int col = tn * BN + e % BN;
+  float* dst = C + static_cast<long long>(row) * N + col;
+  if constexpr (!EDGE) {
+    *reinterpret_cast<floatx4*>(dst) = v;
+  } else if (row < M) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (col + q < N) dst[q] = v[q];
+  }
+}
+
+template <int BM, int BN>
+void launch_sk_fixup(const float* rec, float* C, int M, int N, int tiles_m, int tiles_n, int tail,
+                     const SkPlan& plan, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(tail), BM * BN / 1024);
+  if (M % BM == 0 && N % BN == 0 && N % 4 == 0)
+    gemm_sk_fixup_kernel<BM, BN, false><<<grid, 256, 0, stream>>>(rec, C, M, N, tiles_m, tiles_n, plan);
+  else
+    gemm_sk_fixup_kernel<BM, BN, true><<<grid, 256, 0, stream>>>(rec, C, M, N, tiles_m, tiles_n, plan);
+  ENG_LAUNCH_CHECK();
+}
+
+}  // namespace
+}  // namespace eng

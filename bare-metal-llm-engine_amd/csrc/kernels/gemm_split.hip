@@ -1,0 +1,792 @@
+// gemm_split.hip -- FP32 GEMM on the bf16 matrix cores.
+//
+//   C[M x N] = A[M x K] . B, B fp32 or fp16, given [K x N] or (BNK) [N x K].
+//
+// v_mfma_f32_32x32x16_bf16 runs 16 times the rate of v_mfma_f32_32x32x2_f32.
+// Every fp32 value is the exact sum of three bf16 terms (a = a1 + a2 + a3:
+// a1 = bf16(a), a2 = bf16(a - a1), a3 = a - a1 - a2, 8 bits each), products of
+// two bf16 values are exact in fp32, and the sums accumulate in fp32. Of the
+// nine term products six are taken -- (1,1) (1,2) (2,1) (2,2) (1,3) (3,1); the
+// three left out are at most 2^-23 of |a b| together and 1.4e-8 of it in the
+// root mean square, below half an fp32 rounding. An fp16 B is two terms and
+// all six products. So a 16-deep slice takes six roundings of the running sum
+// where the FP32 instruction takes eight.
+//
+// What the split does not hold is found and done again: a value whose third
+// remainder still has bits below bf16's (a value under 2^-110) sets a flag
+// while it is staged, and infinities, NaN and sums past the fp32 range leave a
+// non-finite accumulator. A workgroup that sees the latter, or the former where
+// it could matter next to its sums, recomputes its tile with
+// v_mfma_f32_32x32x2_f32 on the unsplit operands (4096^3 with one NaN 2.3 ms;
+// with probabilities down to e^-87, flagged everywhere, 0.88 ms).
+//
+// What bounds it: the matrix cores at the clock the card holds under them
+// (4096^3: matrix cores busy 72% of the cycles at about 1.75 GHz; chains of
+// this instruction on random registers sustain 1594 TFLOP/s, 266 of these six-
+// product FLOP), then LDS. 4096^3: 908 -> 629 us (151 -> 218 TFLOP/s) against
+// the FP32 instruction, error against float64 1.1e-6 -> 1.0e-6; 512 x 4096 x
+// 4096 120 -> 95 us; 509 x 2051 x 1023 (no row aligned) 64 -> 29.6 us.
+#include "gemm_plan.hpp"
+#include "device_sync.hpp"
+#include "launch.hpp"
+
+#include <algorithm>
+#include <type_traits>
+#include <utility>
+
+namespace eng {
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+
+constexpr int BK = 32;
+
+// Tile BM x BN by KG groups of WGM x WGN waves; each group takes every KG-th
+// K tile with LDS stages of its own, and the groups' sums are added through
+// LDS at the end.
+template <int BM_, int BN_, int WGM_, int WGN_, int KG_ = 1>
+struct SplitCfg {
+  static constexpr int BM = BM_;
+  static constexpr int BN = BN_;
+  static constexpr int WGM = WGM_;
+  static constexpr int WGN = WGN_;
+  static constexpr int KG = KG_;
+  static constexpr int kGroup = 64 * WGM * WGN;  // threads of a group
+  static constexpr int kThreads = kGroup * KG;
+  static constexpr int WM = BM / WGM;
+  static constexpr int WN = BN / WGN;
+  static constexpr int MB = WM / 32;
+  static constexpr int NB = WN / 32;
+  static constexpr int A8 = BM * BK / 8 / kGroup;  // 8-value chunks a thread stages per K tile
+  static constexpr int B8 = BN * BK / 8 / kGroup;
+  static constexpr int kLds = KG * 2 * 3 * 2 * BK * (BM + BN);
+  // workgroups a CU holds: by LDS, and at most two waves per SIMD (256 registers each)
+  static constexpr int kPerCuLds = 160 * 1024 / kLds;
+  static constexpr int kPerCuWaves = 512 / kThreads;
+  static constexpr int kPerCu = kPerCuLds < kPerCuWaves ? kPerCuLds : kPerCuWaves;
+  static_assert(A8 * 8 * kGroup == BM * BK && B8 * 8 * kGroup == BN * BK, "staging shape");
+  static_assert(KG <= 2 && kPerCu >= 1, "workgroup shape");
+};
+template <typename C>
+using SplitAcc = floatx16[C::MB][C::NB];
+
+// LDS tiles are bf16 planes. Rows along k (A, [N x K] B): 64 bytes, chunk c (8
+// values) of row r at c ^ ((r >> 2) & 3). [K x N] B: rows of BN values, chunk
+// c of row k at c ^ swz_kn<BN>(k), so the 8 rows x 64 bytes a transposing read
+// touches cover the banks twice, the minimum.
+__device__ __forceinline__ int swz_rows(int r) { return (r >> 2) & 3; }
+template <int BN>
+__device__ __forceinline__ int swz_kn(int k) {
+  return BN >= 128 ? 4 * (k & 3) : 4 * ((k >> 1) & 1);
+}
+
+// f(integral_constant<int, I>{}) for each I.
+template <typename F, int... I>
+__device__ __forceinline__ void each_index(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+// Eight values as three bf16 planes; flag collects the bits left in the third
+// remainder (its low half must be empty for the three terms to hold the value).
+__device__ __forceinline__ void split3(const float (&v)[8], uintx4 (&p)[3], unsigned& flag) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const floatx2 x = {v[2 * i], v[2 * i + 1]};
+    const unsigned p1 = __builtin_bit_cast(unsigned, __builtin_convertvector(x, bf16x2));
+    const floatx2 r = {x[0] - __builtin_bit_cast(float, p1 << 16),
+                       x[1] - __builtin_bit_cast(float, p1 & 0xffff0000u)};
+    const unsigned p2 = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+    const unsigned s0 = __builtin_bit_cast(unsigned, r[0] - __builtin_bit_cast(float, p2 << 16));
+    const unsigned s1 =
+        __builtin_bit_cast(unsigned, r[1] - __builtin_bit_cast(float, p2 & 0xffff0000u));
+#if defined(__HIP_DEVICE_COMPILE__)
+    // (in asm: the compiler sinks a plain |= and keeps every remainder live)
+    asm("v_or3_b32 %0, %0, %1, %2" : "+v"(flag) : "v"(s0), "v"(s1));
+#else
+    flag |= s0 | s1;
+#endif
+    p[0][i] = p1;
+    p[1][i] = p2;
+    p[2][i] = __builtin_amdgcn_perm(s1, s0, 0x07060302u);
+  }
+}
+
+// Eight consecutive elements at p as floats. VEC: 16-byte aligned; else only
+// element-aligned (global memory takes dword-aligned 16-byte loads).
+struct __attribute__((packed, aligned(4))) Float4U {
+  float v[4];
+};
+struct __attribute__((packed, aligned(2))) Half8U {
+  _Float16 v[8];
+};
+template <bool VEC, typename T>
+__device__ __forceinline__ void load8(const T* p, float (&v)[8]) {
+  if constexpr (std::is_same<T, float>::value) {
+    if constexpr (VEC) {
+      const floatx4 a = *reinterpret_cast<const floatx4*>(p);
+      const floatx4 b = *reinterpret_cast<const floatx4*>(p + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = a[e], v[4 + e] = b[e];
+    } else {
+      const Float4U a = *reinterpret_cast<const Float4U*>(p);
+      const Float4U b = *reinterpret_cast<const Float4U*>(p + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = a.v[e], v[4 + e] = b.v[e];
+    }
+  } else {
+    if constexpr (VEC) {
+      const halfx8 h = *reinterpret_cast<const halfx8*>(p);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(h[e]);
+    } else {
+      const Half8U h = *reinterpret_cast<const Half8U*>(p);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(h.v[e]);
+    }
+  }
+}
+
+// Operand forms. ALIGNED: K % 32 == 0, 16-byte aligned rows, and [K x N] B with N %
+// 8 == 0. ANY: any K and element alignment ([K x N] B: N % 8 == 0). SHIFT: [K x N]
+// B with any N >= 8: the last column chunk of a row, when it crosses N, is
+// read 8 columns before the row's end and shifted into place.
+enum Form { ALIGNED, ANY, SHIFT };
+
+// The K tiles [kt0, kt1) of the tile at (m0, n0) into acc (zeroed here). With
+// two groups only group 0's acc is the sum.
+template <typename C, bool BNK, typename BT, Form FORM>
+__device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT* __restrict__ B,
+                                           int M, int N, int K, int m0, int n0, int kt0, int kt1,
+                                           SplitAcc<C>& acc) {
+  constexpr int MB = C::MB;
+  constexpr int NB = C::NB;
+  constexpr int A8 = C::A8;
+  constexpr int B8 = C::B8;
+  constexpr int T = C::kGroup;
+  constexpr int KG = C::KG;
+  constexpr int BN = C::BN;
+  constexpr int AP = C::BM * BK;  // bf16 values of one A plane tile
+  constexpr int BP = C::BN * BK;
+  constexpr bool HB = std::is_same<BT, _Float16>::value;
+  constexpr int PB = HB ? 2 : 3;  // B planes
+  constexpr bool GEN = FORM != ALIGNED;
+  __shared__ __attribute__((aligned(1024))) __bf16 As0[KG * 3 * AP];
+  __shared__ __attribute__((aligned(1024))) __bf16 As1[KG * 3 * AP];
+  __shared__ __attribute__((aligned(1024))) __bf16 Bs0[KG * PB * BP];
+  __shared__ __attribute__((aligned(1024))) __bf16 Bs1[KG * PB * BP];
+  __shared__ int wave_bad[C::kThreads / 64];
+
+  const int t = threadIdx.x % T;
+  const int lane = t & 63;
+  const int wg_wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int group = KG == 1 ? 0 : wg_wave / (T / 64);
+  const int wave = wg_wave % (T / 64);
+  const int li = lane & 31;
+  const int lg = lane >> 5;
+  const int wm = wave / C::WGN;
+  const int wn = wave % C::WGN;
+  constexpr int CPR = BNK ? 4 : BN / 8;  // chunks per B tile row
+  auto a_stage = [&](auto st) -> __bf16* {
+    if constexpr (decltype(st)::value == 0) return As0 + group * 3 * AP;
+    else return As1 + group * 3 * AP;
+  };
+  auto b_stage = [&](auto st) -> __bf16* {
+    if constexpr (decltype(st)::value == 0) return Bs0 + group * PB * BP;
+    else return Bs1 + group * PB * BP;
+  };
+
+  // Chunk j of thread t: slot q = T j + t; A and [N x K] B: row q / 4, k chunk
+  // q % 4; [K x N] B: k row q / CPR, column chunk q % CPR. Rows past the
+  // matrix read the last one and columns past it the last chunk: they feed
+  // only elements of C that are not stored.
+  const float* ap[A8];
+  const BT* bp[B8];
+#pragma unroll
+  for (int j = 0; j < A8; ++j) {
+    const int q = T * j + t;
+    ap[j] = A + static_cast<long long>(min(m0 + (q >> 2), M - 1)) * K + 8 * (q & 3);
+  }
+  [[maybe_unused]] int shift[FORM == SHIFT ? B8 : 1];
+#pragma unroll
+  for (int j = 0; j < B8; ++j) {
+    const int q = T * j + t;
+    if constexpr (BNK) {
+      bp[j] = B + static_cast<long long>(min(n0 + (q >> 2), N - 1)) * K + 8 * (q & 3);
+    } else {
+      const int c = n0 + 8 * (q % CPR);
+      if constexpr (FORM == SHIFT) shift[j] = c < N && c + 8 > N ? c + 8 - N : 0;
+      bp[j] = B + static_cast<long long>(q / CPR) * N + min(c, N - 8);
+    }
+  }
+
+  // Chunks 0 .. A8 - 1 are A's, the rest B's: loaded to raw[ch], then split
+  // into the planes.
+  constexpr int CH = A8 + B8;
+  float raw[CH][8];
+  auto load = [&](auto chc, int kt, float(&v)[8]) {
+    constexpr int ch = decltype(chc)::value;
+    const long long k0 = static_cast<long long>(kt) * BK;
+    if constexpr (ch < A8) load8<!GEN>(ap[ch] + k0, v);
+    else load8<!GEN>(bp[ch - A8] + (BNK ? k0 : k0 * N), v);
+  };
+  // The partial K tile, element by element (elements past K are zeros).
+  [[maybe_unused]] auto load_partial = [&](auto chc, int kt, float(&v)[8]) {
+    constexpr int ch = decltype(chc)::value;
+    constexpr bool IS_A = ch < A8;
+    constexpr int j = IS_A ? ch : ch - A8;
+    const int q = T * j + t;
+    const int k0 = kt * BK;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int k = IS_A || BNK ? k0 + 8 * (q & 3) + e : k0 + q / CPR;
+      float w;
+      if constexpr (IS_A) {
+        w = A[static_cast<long long>(min(m0 + (q >> 2), M - 1)) * K + min(k, K - 1)];
+      } else if constexpr (BNK) {
+        w = static_cast<float>(
+            B[static_cast<long long>(min(n0 + (q >> 2), N - 1)) * K + min(k, K - 1)]);
+      } else {
+        w = static_cast<float>(
+            B[static_cast<long long>(min(k, K - 1)) * N + min(n0 + 8 * (q % CPR) + e, N - 1)]);
+      }
+      v[e] = k < K ? w : 0.0f;
+    }
+  };
+  unsigned flag = 0;
+  // (whole: v as load() leaves it, else as load_partial() does)
+  auto put = [&](auto chc, __bf16* as, __bf16* bs, float(&v)[8], auto whole) {
+    constexpr int ch = decltype(chc)::value;
+    constexpr bool IS_A = ch < A8;
+    const int q = T * (IS_A ? ch : ch - A8) + t;
+    if constexpr (!IS_A && FORM == SHIFT && decltype(whole)::value) {
+#pragma unroll
+      for (int b = 4; b > 0; b >>= 1) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float here = v[e];
+          const float there = v[e + b < 8 ? e + b : e];
+          v[e] = (shift[ch - A8] & b) ? there : here;
+        }
+      }
+    }
+    uintx4 p[3];
+    split3(v, p, flag);
+    if constexpr (IS_A) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        *reinterpret_cast<uintx4*>(as + i * AP + (q >> 2) * BK + 8 * ((q & 3) ^ swz_rows(q >> 2))) =
+            p[i];
+    } else {
+      const int off = BNK ? (q >> 2) * BK + 8 * ((q & 3) ^ swz_rows(q >> 2))
+                          : (q / CPR) * BN + 8 * ((q % CPR) ^ swz_kn<BN>(q / CPR));
+#pragma unroll
+      for (int i = 0; i < PB; ++i) *reinterpret_cast<uintx4*>(bs + i * BP + off) = p[i];
+    }
+  };
+  auto each_chunk = [&](auto f) { each_index(f, std::make_integer_sequence<int, CH>{}); };
+
+  struct Slice {
+    bf16x8 a[3][MB];
+    bf16x8 b[PB][NB];
+  };
+  auto read_s = [&](const __bf16* as, const __bf16* bs, int sl, Slice& f) {
+    const int cq = 2 * sl + lg;  // this lane's chunk: k = 16 sl + 8 lg .. + 7
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const int r = wm * C::WM + mb * 32 + li;
+        f.a[p][mb] =
+            *reinterpret_cast<const bf16x8*>(as + p * AP + r * BK + 8 * (cq ^ swz_rows(r)));
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        if constexpr (BNK) {
+          const int r = wn * C::WN + nb * 32 + li;
+          f.b[p][nb] =
+              *reinterpret_cast<const bf16x8*>(bs + p * BP + r * BK + 8 * (cq ^ swz_rows(r)));
+        } else {
+          // Two transposing reads per fragment (ds_read_b64_tr_b16): in each
+          // 16-lane group lane l names 8 bytes (row k0 + l / 4, columns cb + 4
+          // (l % 4) .. + 3) and receives column cb + l of the 4 rows.
+          const int l = lane & 15;
+          const int G = lane >> 4;
+          const int col = wn * C::WN + nb * 32 + 16 * (G & 1) + 4 * (l & 3);
+          uintx4 w;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int k = 16 * sl + 8 * (G >> 1) + 4 * h + (l >> 2);
+            const int off = k * (BN * 2) + (((col >> 3) ^ swz_kn<BN>(k)) << 4) + ((col & 7) << 1);
+            const uintx2 v = __builtin_bit_cast(
+                uintx2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (__attribute__((address_space(3))) shortx4*)(
+                                (__attribute__((address_space(3))) char*)(bs + p * BP) + off)));
+            w[2 * h] = v[0];
+            w[2 * h + 1] = v[1];
+          }
+          f.b[p][nb] = __builtin_bit_cast(bf16x8, w);
+        }
+      }
+    }
+  };
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mb][nb][v] = 0.0f;
+  // MFMAs [lo, hi) of a slice's 6 MB NB, by product, then block.
+  constexpr int NM = 6 * MB * NB;
+  auto mma = [&](const Slice& f, int lo, int hi) {
+    constexpr int P[6][2] = {{2, 0}, {HB ? 2 : 0, HB ? 1 : 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const int n = (i * MB + mb) * NB + nb;
+          if (n >= lo && n < hi)
+            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                f.a[P[i][0]][mb], f.b[P[i][1]][nb], acc[mb][nb], 0, 0, 0);
+        }
+    }
+  };
+
+  // One K tile per step from stage st: the tile's second slice is read while
+  // the first is multiplied, and the next tile's planes (its values loaded a
+  // step ago) are written to the other stage and the loads of the tile after
+  // it issued meanwhile; one barrier, then the next tile's first slice is read
+  // while the second is multiplied. Past the end the last tile is staged
+  // again, never used. The scheduling groups put each chunk's split (about 50
+  // vector instructions) behind its share of the MFMAs, which leave the vector
+  // unit free for most of their 32 cycles.
+  [[maybe_unused]] constexpr int READS = 3 * MB + PB * NB * (BNK ? 1 : 2);  // fragment reads of a slice
+  Slice x, y;
+  auto step = [&](auto st, int next_kt) {
+    using Next = std::integral_constant<int, 1 - decltype(st)::value>;
+    read_s(a_stage(st), b_stage(st), 1, y);
+    each_chunk([&](auto chc) {
+      constexpr int ch = decltype(chc)::value;
+      put(chc, a_stage(Next{}), b_stage(Next{}), raw[ch], std::true_type{});
+      load(chc, next_kt, raw[ch]);
+      mma(x, ch * NM / CH, (ch + 1) * NM / CH);
+#if defined(__HIP_DEVICE_COMPILE__)
+      constexpr int n = (ch + 1) * NM / CH - ch * NM / CH;
+      constexpr int reads = ch == 0 ? (READS + n - 1) / n : 0;
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                             // an MFMA
+        if constexpr (reads > 0) __builtin_amdgcn_sched_group_barrier(0x100, reads, 0);  // LDS reads
+        __builtin_amdgcn_sched_group_barrier(0x002, (52 + n - 1) / n, 0);              // the split
+      }
+      __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);  // plane writes
+      __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);  // the loads
+      __builtin_amdgcn_sched_barrier(0);
+#endif
+    });
+    lds_barrier();
+    read_s(a_stage(Next{}), b_stage(Next{}), 0, x);
+    mma(y, 0, NM);
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int per = (2 * READS + NM - 1) / NM;
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#pragma unroll
+    for (int i = 0; i < (READS + per - 1) / per; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x100, per, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  // n whole K tiles per group in the pipeline (group g: kt0 + g, kt0 + g + KG,
+  // ...); the rest -- whole tiles left over, the partial one, and every tile of
+  // an N below one chunk -- staged and multiplied one by one.
+  const int whole_end = GEN ? (FORM == SHIFT && N < 8 ? 0 : K / BK) : kt1;
+  const int n = max(min(kt1, whole_end) - kt0, 0) / KG;
+  const int first = kt0 + group;
+  const int last = first + (n - 1) * KG;
+  auto put_all = [&](auto whole) {
+    each_chunk([&](auto c) {
+      put(c, a_stage(I0{}), b_stage(I0{}), raw[decltype(c)::value], whole);
+    });
+  };
+  if (n > 0) {
+    each_chunk([&](auto c) { load(c, first, raw[decltype(c)::value]); });
+    put_all(std::true_type{});
+    each_chunk([&](auto c) { load(c, min(first + KG, last), raw[decltype(c)::value]); });
+    lds_barrier();
+    read_s(a_stage(I0{}), b_stage(I0{}), 0, x);
+    int i = 0;
+    for (; i + 1 < n; i += 2) {
+      step(I0{}, min(first + (i + 2) * KG, last));
+      step(I1{}, min(first + (i + 3) * KG, last));
+    }
+    if (i < n) step(I0{}, last);
+  }
+#pragma unroll 1
+  for (int k = kt0 + n * KG; k < kt1; k += KG) {
+    const int kt = k + group;
+    __syncthreads();  // every wave has read the stages
+    if (kt < kt1) {
+      if (GEN && kt >= whole_end) {
+        each_chunk([&](auto c) { load_partial(c, kt, raw[decltype(c)::value]); });
+        put_all(std::false_type{});
+      } else {
+        each_chunk([&](auto c) { load(c, kt, raw[decltype(c)::value]); });
+        put_all(std::true_type{});
+      }
+    }
+    __syncthreads();
+    if (kt < kt1) {
+      read_s(a_stage(I0{}), b_stage(I0{}), 0, x);
+      read_s(a_stage(I0{}), b_stage(I0{}), 1, y);
+      mma(x, 0, NM);
+      mma(y, 0, NM);
+    }
+  }
+
+  // Non-finite sums (bit 0) and values the three terms do not hold (bit 1).
+  bool inf = false;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) inf |= !(fabsf(acc[mb][nb][v]) <= 3.4028235e38f);
+  const int wave_any = (__ballot(inf) != 0 ? 1 : 0) | (__ballot((flag & 0xffffu) != 0) != 0 ? 2 : 0);
+  if (lane == 0) wave_bad[wg_wave] = wave_any;
+  __syncthreads();
+  int any = 0;
+#pragma unroll
+  for (int w = 0; w < C::kThreads / 64; ++w) any |= wave_bad[w];
+  bool again = (any & 1) != 0;
+  if constexpr (KG == 2) {
+    static_assert(KG * 3 * AP * 2 >= C::BM * C::BN * 4, "the sums fit the A stage");
+    float* red = reinterpret_cast<float*>(As0) + wave * (MB * NB * 16 * 64) + lane;
+    // (after the barrier above every wave has read its stages)
+    if (group == 1) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) red[((mb * NB + nb) * 16 + v) * 64] = acc[mb][nb][v];
+    }
+    __syncthreads();
+    if (group == 0) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[mb][nb][v] += red[((mb * NB + nb) * 16 + v) * 64];
+    }
+    __syncthreads();  // a following tile may refill the stages
+  }
+  const int k0 = kt0 * BK;
+  const int k1 = min(kt1 * BK, K);
+  if (!again && any != 0) {
+    // A value the terms do not hold is off by at most 2^-133, so the sums by
+    // (k1 - k0) 2^-133 (max |a| + max |b|): nothing next to any sum of ordinary
+    // size (tiny probabilities beside large ones), and otherwise again.
+    float amax = 0.0f, bmax = 0.0f, least = 3.4028235e38f;
+    constexpr int W = C::kThreads / 64;
+    // a row's values along k, 8 loads in flight per lane (past the end
+    // the last value again)
+    auto row_max = [&](const auto* row, float m) {
+      for (int k = k0 + lane; k < k1; k += 8 * 64) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = static_cast<float>(row[min(k + 64 * u, k1 - 1)]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) m = fmaxf(m, fabsf(v[u]));
+      }
+      return m;
+    };
+    for (int r = wg_wave; r < C::BM; r += W)
+      amax = row_max(A + static_cast<long long>(min(m0 + r, M - 1)) * K, amax);
+    if constexpr (BNK) {
+      for (int r = wg_wave; r < BN; r += W)
+        bmax = row_max(B + static_cast<long long>(min(n0 + r, N - 1)) * K, bmax);
+    } else {
+      for (int k = k0 + 8 * wg_wave; k < k1; k += 8 * W) {
+        float v[8][BN / 64];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int c = 0; c < BN / 64; ++c)
+            v[u][c] = static_cast<float>(B[static_cast<long long>(min(k + u, k1 - 1)) * N +
+                                           min(n0 + 64 * c + lane, N - 1)]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int c = 0; c < BN / 64; ++c) bmax = fmaxf(bmax, fabsf(v[u][c]));
+      }
+    }
+    if (group == 0) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) least = fminf(least, fabsf(acc[mb][nb][v]));
+    }
+    float* wave_max = reinterpret_cast<float*>(As0);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      amax = fmaxf(amax, __shfl_xor(amax, o));
+      bmax = fmaxf(bmax, __shfl_xor(bmax, o));
+      least = fminf(least, __shfl_xor(least, o));
+    }
+    if (lane == 0) {
+      wave_max[3 * wg_wave] = amax;
+      wave_max[3 * wg_wave + 1] = bmax;
+      wave_max[3 * wg_wave + 2] = least;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      amax = fmaxf(amax, wave_max[3 * w]);
+      bmax = fmaxf(bmax, wave_max[3 * w + 1]);
+      least = fminf(least, wave_max[3 * w + 2]);
+    }
+    // (2^-67 on both sides: 2^-133 is a subnormal)
+    again = !(static_cast<float>(k1 - k0) * 0x1p-66f * (amax + bmax) * 0x1p-40f <= least * 0x1p+1f);
+    __syncthreads();  // As0 is refilled by a following tile
+  }
+  if (again && group == 0) {
+    // Once more on the FP32 instruction, straight from memory.
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[mb][nb][v] = 0.0f;
+    constexpr int U = 8;  // MFMA steps whose loads are in flight together
+#pragma unroll 1
+    for (int k = kt0 * BK; k < k1; k += 2 * U) {
+      float a[U][MB], b[U][NB];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int ku = k + 2 * u + lg;
+        const int kk = min(ku, K - 1);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          const int r = min(m0 + wm * C::WM + mb * 32 + li, M - 1);
+          const float v = A[static_cast<long long>(r) * K + kk];
+          a[u][mb] = ku < k1 ? v : 0.0f;
+        }
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const int n = min(n0 + wn * C::WN + nb * 32 + li, N - 1);
+          const float v = static_cast<float>(BNK ? B[static_cast<long long>(n) * K + kk]
+                                                 : B[static_cast<long long>(kk) * N + n]);
+          b[u][nb] = ku < k1 ? v : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            acc[mb][nb] =
+                __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][mb], b[u][nb], acc[mb][nb], 0, 0, 0);
+    }
+  }
+}
+
+template <typename C>
+__device__ __forceinline__ void split_store(const SplitAcc<C>& acc, float* __restrict__ out,
+                                            long long ld, int rows_left, int cols_left) {
+  if (C::KG > 1 && threadIdx.x >= C::kGroup) return;  // group 0 holds the sum
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int li = lane & 31;
+  const int lg = lane >> 5;
+  const int wm = wave / C::WGN;
+  const int wn = wave % C::WGN;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(ld));  // keeps the element offsets out of the tile loop's registers
+#endif
+  const bool whole = rows_left >= C::BM && cols_left >= C::BN;
+#pragma unroll
+  for (int mb = 0; mb < C::MB; ++mb) {
+#pragma unroll
+    for (int nb = 0; nb < C::NB; ++nb) {
+      const int col = wn * C::WN + nb * 32 + li;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int row = wm * C::WM + mb * 32 + 8 * (v >> 2) + 4 * lg + (v & 3);
+        if (whole || (row < rows_left && col < cols_left)) out[row * ld + col] = acc[mb][nb][v];
+      }
+    }
+  }
+}
+
+template <typename C, bool BNK, typename BT, Form FORM>
+__global__ __launch_bounds__(C::kThreads, C::kPerCu) void gemm_split_kernel(
+    const float* __restrict__ A, const BT* __restrict__ B, float* __restrict__ out,
+    float* __restrict__ rec, int M, int N, int K, int tiles_m, int tiles_n, SkPlan plan) {
+  const int g = blockIdx.x;
+  const bool dp = g < plan.dp;
+  const long long s = dp ? 0 : g - plan.dp;
+  const long long i0 = dp ? 0 : sk_begin(s, plan);
+  const long long i1 = dp ? plan.nk : sk_begin(s + 1, plan);
+  const int first_tile = dp ? g : plan.dp;
+  SplitAcc<C> acc;
+  for (long long it = i0; it < i1;) {
+    const long long t = it / plan.nk;
+    const int ka = static_cast<int>(it - t * plan.nk);
+    const long long tend = (t + 1) * plan.nk;
+    const int kb = static_cast<int>((i1 < tend ? i1 : tend) - t * plan.nk);
+    int tm, tn;
+    tile_of(first_tile + static_cast<int>(t), tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * C::BM;
+    const int n0 = tn * C::BN;
+    split_tile<C, BNK, BT, FORM>(A, B, M, N, K, m0, n0, ka, kb, acc);
+    if (ka == 0 && kb == plan.nk) {
+      split_store<C>(acc, out + static_cast<long long>(m0) * N + n0, N, M - m0, N - n0);
+    } else {
+      const int slot = it == i0 ? 0 : 1;
+      split_store<C>(acc, rec + (s * 2 + slot) * static_cast<long long>(C::BM * C::BN), C::BN, C::BM,
+                     C::BN);
+    }
+    it = t * plan.nk + kb;
+  }
+}
+
+// How a call is cut: whole rounds of tiles (one per resident workgroup) run one
+// per workgroup, and the tiles past them either as one more round or, split by
+// K, evenly over up to one workgroup per CU (records and a fix-up pass).
+struct Cut {
+  double us = 0;        // estimated time
+  long long split = 0;  // workgroups sharing the tail tiles (0: not split)
+};
+
+// Estimated time of a tiling: `step` is a workgroup's time per K tile on a full
+// chip, `fill` what a round costs besides (first loads, stores), `rec` what one
+// split workgroup's record adds (written, read back). A split costs the fix-up
+// launch and another fill, about 8 us, and 3 more where workgroups cross from
+// one tile into the next.
+Cut cut_of(long long M, long long N, long long nk, long long bm, long long bn, double step,
+           double fill, double rec, long long cus) {
+  const long long tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  const long long tail = tiles % cus;
+  const double round = static_cast<double>(nk) * step + fill;
+  Cut c;
+  c.us = static_cast<double>((tiles + cus - 1) / cus) * round;
+  if (tail != 0 && nk >= 16 && tiles < 2 * cus) {
+    // at least 8 K tiles each
+    const long long w = std::max<long long>(tail, std::min(cus, tail * nk / 8));
+    const double us = static_cast<double>(tiles / cus) * round + fill +
+                      static_cast<double>(tail * nk) / static_cast<double>(w) * step + 8.0 +
+                      rec * static_cast<double>(w) + (w % tail != 0 ? 3.0 : 0.0);
+    if (w > tail && us < c.us) c.us = us, c.split = w;
+  }
+  return c;
+}
+
+template <typename C, typename BT, bool BNK>
+void run_split(const GemmArgs& a, Form form, const Cut& cut, long long cus, hipStream_t stream) {
+  const int M = static_cast<int>(a.M), N = static_cast<int>(a.N), K = static_cast<int>(a.K);
+  const int tiles_m = (M + C::BM - 1) / C::BM;
+  const int tiles_n = (N + C::BN - 1) / C::BN;
+  const long long ntiles = static_cast<long long>(tiles_m) * tiles_n;
+  ENG_CHECK(ntiles <= 0x7fffffffLL, "matmul: too many tiles for one launch");
+  SkPlan plan;
+  plan.nk = (K + BK - 1) / BK;
+  const long long tail = cut.split > 0 ? ntiles % cus : 0;
+  plan.dp = static_cast<int>(ntiles - tail);
+  plan.I = tail * plan.nk;
+  plan.nsk = static_cast<int>(tail > 0 ? cut.split : 0);
+  const BT* B = static_cast<const BT*>(a.B);
+  auto launch = [&](auto f, float* rec) {
+    gemm_split_kernel<C, BNK, BT, decltype(f)::value>
+        <<<dim3(static_cast<unsigned>(plan.dp + plan.nsk)), C::kThreads, 0, stream>>>(
+            a.A, B, a.C, rec, M, N, K, tiles_m, tiles_n, plan);
+    ENG_LAUNCH_CHECK();
+  };
+  auto go = [&](float* rec) {
+    if constexpr (std::is_same<BT, float>::value) {
+      if (form == ALIGNED) return launch(std::integral_constant<Form, ALIGNED>{}, rec);
+    }
+    if constexpr (!BNK) {
+      if (form == SHIFT) return launch(std::integral_constant<Form, SHIFT>{}, rec);
+    }
+    launch(std::integral_constant<Form, ANY>{}, rec);
+  };
+  if (tail == 0) {
+    go(nullptr);
+    return;
+  }
+  StreamScratch records(
+      stream, static_cast<std::size_t>(plan.nsk) * 2 * C::BM * C::BN * sizeof(float), 2);
+  float* rec = static_cast<float*>(records.get());
+  go(rec);
+  launch_sk_fixup<C::BM, C::BN>(rec, a.C, M, N, tiles_m, tiles_n, static_cast<int>(tail), plan,
+                                stream);
+}
+
+// The tiling of the smallest estimated time. Microseconds per K tile and
+// workgroup, measured with every CU busy (4096^3, 2048^3 and 512 x 4096 x 4096):
+//   256 x 128, 8 waves of 64 x 64                2.46  (4096^3: 629 us, 218 TFLOP/s)
+//   128 x 128, 8 waves of 64 x 32                1.39  (2048^3: 91 us, 189 TFLOP/s)
+//   128 x 64, two groups of 4 waves of 64 x 32   0.83  (512 x 4096 x 4096: 104 us)
+//   64 x 64, two groups of 4 waves of 32 x 32    0.52  (1024^3: 20 us)
+// against the FP32 instruction's kernels (fp32_us), which stay ahead where one
+// round of their small tiles holds the whole call (1024^3: 17.9 us, 512^3: 5.6).
+template <typename BT, bool BNK>
+bool split_dispatch(const GemmArgs& a, double fp32_us, long long cus, hipStream_t stream) {
+  constexpr int kBVec = 16 / static_cast<int>(sizeof(BT));
+  Form form = ALIGNED;
+  if (!BNK && a.N % 8 != 0)
+    form = SHIFT;
+  else if (a.K % BK != 0 || !aligned_to(a.A, 16) || !aligned_to(a.B, 16) ||
+           (BNK ? a.K : a.N) % kBVec != 0)
+    form = ANY;
+  const long long nk = (a.K + BK - 1) / BK;
+  const double part = a.K % BK != 0 ? 1.5 : 0.0;  // the partial K tile, by itself
+  const Cut big = cut_of(a.M, a.N, nk, 256, 128, 2.46, 5.0 + part, 0.05, cus);
+  const Cut mid = cut_of(a.M, a.N, nk, 128, 128, 1.39, 3.5 + part, 0.02, cus);
+  const Cut low = cut_of(a.M, a.N, nk, 128, 64, 0.83, 3.0 + part, 0.01, cus);
+  const Cut sml = cut_of(a.M, a.N, nk, 64, 64, 0.52, 2.0 + part, 0.005, cus);
+  const double best = std::min(std::min(big.us, mid.us), std::min(low.us, sml.us));
+  if (fp32_us <= best) return false;
+  if (big.us == best)
+    run_split<SplitCfg<256, 128, 4, 2>, BT, BNK>(a, form, big, cus, stream);
+  else if (mid.us == best)
+    run_split<SplitCfg<128, 128, 2, 4>, BT, BNK>(a, form, mid, cus, stream);
+  else if (low.us == best)
+    run_split<SplitCfg<128, 64, 2, 2, 2>, BT, BNK>(a, form, low, cus, stream);
+  else
+    run_split<SplitCfg<64, 64, 2, 2, 2>, BT, BNK>(a, form, sml, cus, stream);
+  return true;
+}
+
+}  // namespace
+
+bool launch_gemm_split(const GemmArgs& a, double fp32_us, long long cus, hipStream_t stream) {
+  if (a.b == Elem::F32)
+    return a.b_nk ? split_dispatch<float, true>(a, fp32_us, cus, stream)
+                  : split_dispatch<float, false>(a, fp32_us, cus, stream);
+  return a.b_nk ? split_dispatch<_Float16, true>(a, fp32_us, cus, stream)
+                : split_dispatch<_Float16, false>(a, fp32_us, cus, stream);
+}
+
+}  // namespace eng

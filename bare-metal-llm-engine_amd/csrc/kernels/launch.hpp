@@ -158,6 +158,10 @@ struct GemmArgs {
   std::int64_t K = 0;
 };
 void launch_gemm(const GemmArgs& a, hipStream_t stream);
+// The same product on the bf16 matrix cores (gemm_split.hip). Returns false,
+// launching nothing, when it estimates more than `fp32_us` microseconds (the
+// caller's own estimate). cus: device_cu_count().
+bool launch_gemm_split(const GemmArgs& a, double fp32_us, long long cus, hipStream_t stream);
 
 // out[r][c] = in[r][c] * s_r * weight[c] (weight optional).
 void launch_rmsnorm(const float* in, const float* weight, float* out, long long rows,

@@ -1,0 +1,115 @@
+"""The FP32 GEMM on the bf16 matrix cores (three exact bf16 terms per value):
+every tile shape and operand form at ragged sizes, exact products where the
+three terms must hold them, and the values the terms do not hold (infinities,
+NaN, tiny and largest values), which the kernel recomputes on the FP32
+instruction.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import helpers
+
+pytestmark = pytest.mark.gpu
+U = helpers.U32
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    helpers.ensure_built()
+    return helpers.load_package().Engine()
+
+
+def gemm(gpu, A, B):
+    dA, dB = gpu.upload(A), gpu.upload(B)
+    dC = gpu.empty((A.shape[0], B.shape[1]), np.float32)
+    dC.fill_bytes(0xFF)
+    gpu.call("eng_matmul_f32", dA.ptr, dB.ptr, dC.ptr, A.shape[0], B.shape[1], A.shape[1], None)
+    gpu.sync()
+    return dC.download()
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1536, 4096, 512),    # 256 x 128 tiles, whole
+    (1531, 4093, 515),    # ... every edge ragged, a partial K tile, columns shifted into place
+    (2048, 2048, 512),    # 128 x 128
+    (2041, 2056, 530),    # ... ragged, N a multiple of 8
+    (512, 4096, 1000),    # K split over workgroups (records and the fix-up pass)
+    (509, 2051, 1023),    # 128 x 64 in two K groups
+    (130, 250, 1000),     # 64 x 64 in two K groups
+    (129, 257, 993),      # ... one column past a tile, 31 whole K tiles and one value
+    (300, 999, 4000),     # small tiles split over K
+    (4096, 5, 300),       # N below one column chunk
+    (100, 3, 700),
+    (65, 8, 1001),
+])
+def test_split_gemm_against_float64(gpu, M, N, K):
+    rng = np.random.default_rng(M + 3 * N + 7 * K)
+    A = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    got = gemm(gpu, A, B)
+    y64 = helpers.as_f64(A) @ helpers.as_f64(B)
+    derived, stat = helpers.dot_bounds(helpers.absdot(A, B), y64, K)
+    helpers.assert_within(got, y64, np.minimum(derived, stat), f"{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("M,N,K", [(1531, 1024, 1024), (300, 999, 999)])
+def test_split_gemm_times_identity_is_exact(gpu, M, N, K):
+    """A . I = A bit for bit: the three terms of a value add up to it, over 200
+    binary orders of magnitude."""
+    rng = np.random.default_rng(3)
+    A = (rng.uniform(1, 2, (M, K)) * 2.0 ** rng.integers(-100, 100, (M, K))).astype(np.float32)
+    A *= rng.choice(np.float32([-1, 1]), A.shape)
+    B = np.zeros((K, N), np.float32)
+    B[np.arange(min(K, N)), np.arange(min(K, N))] = 1.0
+    got = gemm(gpu, A, B)
+    assert np.array_equal(got[:, :min(K, N)], A[:, :min(K, N)])
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 1024, 704), (300, 999, 701), (1536, 4096, 512)])
+def test_split_gemm_infinities_nan_and_extreme_values(gpu, M, N, K):
+    rng = np.random.default_rng(11)
+    A = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    A[3, 5] = np.inf
+    A[7, 6] = -np.inf
+    A[7, 9] = np.inf        # meets both signs: NaN where the products disagree
+    A[11, K - 1] = np.nan
+    A[130] *= np.float32(1e-37)             # down to fp32 subnormals
+    A[131, ::2] *= np.float32(1e-42)
+    A[140] *= np.float32(1e36)
+    A[141, 17] = np.finfo(np.float32).max   # rounds past bf16's range
+    B[17] *= np.float32(1e-30)
+    B[20, 200] = np.inf
+    B[21, 201] = np.nan
+    B[:, 202] = 0.0
+    got = gemm(gpu, A, B)
+    with np.errstate(invalid="ignore"):
+        y64 = helpers.as_f64(A) @ helpers.as_f64(B)
+    fin = np.isfinite(y64)
+    assert np.array_equal(np.isnan(got), np.isnan(y64))
+    assert np.array_equal(got[~fin & ~np.isnan(y64)], y64[~fin & ~np.isnan(y64)].astype(np.float32))
+    with np.errstate(invalid="ignore"):
+        a = helpers.absdot(A, B)
+    # each of the K products and sums also rounds to at most half of the
+    # smallest subnormal, 2^-150
+    bound = K * U * np.where(fin, a, 0) + U * np.abs(np.where(fin, y64, 0)) + 2 * K * 2.0**-150
+    err = np.abs(np.where(fin, got, 0).astype(np.float64) - np.where(fin, y64, 0))
+    assert (err <= bound).all(), float((err / bound).max())
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 999, 701), (1536, 4096, 512)])
+def test_split_gemm_tiny_values_beside_ordinary_ones(gpu, M, N, K):
+    """Probabilities down to e^-87 (values the three terms do not hold, in every
+    tile) times ordinary values, and rows of nothing but tiny ones."""
+    rng = np.random.default_rng(5)
+    A = np.exp(-rng.uniform(0, 87, (M, K))).astype(np.float32)
+    A[256:290] = A[256:290] * np.float32(1e-36)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    got = gemm(gpu, A, B)
+    y64 = helpers.as_f64(A) @ helpers.as_f64(B)
+    bound = K * U * helpers.absdot(A, B) + U * np.abs(y64) + 2 * K * 2.0**-150
+    err = np.abs(got - y64)
+    assert (err <= bound).all(), float((err / bound).max())
