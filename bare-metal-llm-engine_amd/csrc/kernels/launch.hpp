@@ -126,6 +126,10 @@ bool skinny_applies(const SkinnyArgs& a);
 // Scratch bytes launch_skinny takes (0 when K is not split).
 std::size_t skinny_scratch_bytes(const SkinnyArgs& a);
 void launch_skinny(const SkinnyArgs& a, hipStream_t stream);
+// The same for fp16 W [N x K] with RMSNorm, in one launch (few_rows.hip);
+// applies: for calls skinny_applies takes, whether it is the faster one.
+bool few_rows_nk_applies(const SkinnyArgs& a);
+void launch_few_rows_nk(const SkinnyArgs& a, hipStream_t stream);
 // The few-row form of an M-row GEMV-style call (fp32 x and y only; other
 // element types give M = 0, which no kernel takes).
 inline SkinnyArgs skinny_args(const GemvArgs& g, std::int64_t M) {

@@ -1100,6 +1100,10 @@ std::size_t skinny_scratch_bytes(const SkinnyArgs& a) {
 
 void launch_skinny(const SkinnyArgs& a, hipStream_t stream) {
   ENG_CHECK(skinny_applies(a), "linear: shape not supported by the few-row kernel");
+  if (few_rows_nk_applies(a)) {
+    launch_few_rows_nk(a, stream);
+    return;
+  }
   if (a.w == Elem::F16) {
     if (a.w_nk) {
       dispatch_rms<_Float16, true>(a, stream);

@@ -201,3 +201,33 @@ def test_few_rows_k_zero_and_contracts(gpu):
     gpu.call("eng_rmsnorm_linear_f16w", dA.ptr, None, dA.ptr, dy.ptr, 8, 64, 0, EPS, None)
     gpu.sync()
     assert np.all(dy.download() == 7.0)
+
+
+@pytest.mark.parametrize("N,K", [
+    (10000, 520),    # 48 weight rows per workgroup, the last partly past N; a partial k block
+    (8200, 512),     # one whole block
+    (9999, 3080),    # six blocks in the steady loop, then a partial one
+    (5000, 1536),    # 32 weight rows per workgroup
+    (333, 264),      # 16 weight rows, less than one block
+    (1000, 4104),    # ... eight blocks and 8 values
+])
+@pytest.mark.parametrize("M", [5, 16, 17, 32])
+@pytest.mark.parametrize("with_gamma", [True, False])
+def test_few_rows_one_launch_kernel(gpu, orc, M, N, K, with_gamma):
+    """Output-major fp16 weights over 5-32 rows in one launch, against the oracle,
+    with rows of very different scale in one batch."""
+    rng = np.random.default_rng(N + K + M)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    x *= (10.0 ** rng.integers(-6, 7, (M, 1))).astype(np.float32)
+    x[0, : K // 2] *= np.float32(1e-4)
+    g = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32) if with_gamma else None
+    W = orc.f32_to_f16((rng.standard_normal((K, N), dtype=np.float32) / np.sqrt(K)).astype(np.float32))
+    Wt = np.ascontiguousarray(W.T)
+    dx, dW, dy = gpu.upload(x), gpu.upload(Wt), gpu.empty((M, N), np.float32)
+    dg = gpu.upload(g) if g is not None else None
+    gpu.call("eng_rmsnorm_linear_f16w_nk", dx.ptr, dg.ptr if dg else None, dW.ptr, dy.ptr, M, N, K,
+             1e-5, None)
+    gpu.sync()
+    y = orc.rmsnorm_linear(x, g, W, 1e-5).astype(np.float64)
+    derived, stat = helpers.rmsnorm_linear_bounds(x, g, W, y, K)
+    helpers.assert_within(dy.download(), y, np.minimum(derived, stat), f"{M}x{N}x{K}")
