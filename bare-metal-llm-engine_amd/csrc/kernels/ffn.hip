@@ -20,8 +20,10 @@
 //   * Otherwise gate and up are computed separately into the stream's scratch
 //     arena -- single-row GEMVs, small-batch passes over W, or (more rows)
 //     RMSNorm once and the MFMA GEMM: with fp16 weights (either layout) the
-//     rows are split once into three fp16 planes and gate and up each run the
-//     fp16-MFMA GEMM (launch_gemm_h3) -- and the SwiGLU kernel finishes.
+//     rows are split once into three fp16 planes, and gate and up run either as
+//     one fp16-MFMA GEMM over both with SwiGLU in its stores
+//     (launch_gemm_h3_glu) or each its own (launch_gemm_h3) -- and the SwiGLU
+//     kernel finishes.
 // Preconditions and messages follow rmsnorm_linear; any zero dimension
 // writes nothing.
 #include "gemv_kernels.hpp"
@@ -223,10 +225,6 @@ void rmsnorm_linear_swiglu(const float* in, const float* gamma, const WT* Wg, co
     } else if (!(nk ? launch_gemv_nk_rows(gv, M, s) : launch_gemv_kn_rows(gv, M, s))) {
       // more than a few rows: normalise once, then the MFMA GEMM
       if (h3) {
-        if (!normed) {
-          launch_rmsnorm_split3(in, gamma, planes, rscale, M, K, eps, s);
-          normed = true;
-        }
         GemmH3Args h;
         h.P = planes;
         h.rscale = rscale;
@@ -236,6 +234,13 @@ void rmsnorm_linear_swiglu(const float* in, const float* gamma, const WT* Wg, co
         h.N = N;
         h.K = K;
         h.b_kn = !nk;
+        if (!normed) {
+          launch_rmsnorm_split3(in, gamma, planes, rscale, M, K, eps, s);
+          normed = true;
+          h.C = act;
+          if (launch_gemm_h3_glu(h, reinterpret_cast<const _Float16*>(Wu), s)) return;
+          h.C = out;
+        }
         launch_gemm_h3(h, s);
         continue;
       }

@@ -29,6 +29,7 @@
 // The workgroup -> tile map of every GEMM here is XCD-aware (tile_of).
 #include "gemm_plan.hpp"
 #include "launch.hpp"
+#include "silu.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -795,9 +796,14 @@ __device__ __forceinline__ int swz_h3_kn(int k) { return 4 * (k & 3); }
 // K tiles [kt0, kt1) of the BMT x BNT tile at (m0, n0) into acc (zeroed
 // here); ends with a barrier, so a following call may refill the stages. BKN:
 // B given [K x N] (the reference layout) instead of [N x K].
-template <int S, int BMT, int BNT, bool BKN, bool EDGE>
+// DUAL ([N x K] only): the tile is BNT / 2 columns of two weight matrices B and
+// B2 (the FFN's gate and up), B's rows in LDS ahead of B2's; a wave's column
+// blocks nb = 0 and 1 are the same 32 columns of the two.
+template <int S, int BMT, int BNT, bool BKN, bool EDGE, bool DUAL = false>
 __device__ __forceinline__ void h3_tile(const _Float16* __restrict__ P,
-                                        const _Float16* __restrict__ B, int M, int N, int K,
+                                        const _Float16* __restrict__ B,
+                                        [[maybe_unused]] const _Float16* __restrict__ B2, int M,
+                                        int N, int K,
                                         int m0, int n0, int kt0, int kt1,
                                         h3::Acc<BMT, BNT>& acc) {
   using Sh = h3::Shape<BMT, BNT>;
@@ -813,6 +819,10 @@ __device__ __forceinline__ void h3_tile(const _Float16* __restrict__ P,
   constexpr int LOADS = Sh::LOADS;
   constexpr int AT = 3 * PT;    // halves of a stage's plane tiles
   constexpr int BTL = BNT * BK; // halves of a stage's B tile
+  constexpr int SUB = DUAL ? BNT / 2 : BNT;  // columns of a B (sub-)tile
+  constexpr int SUB_SLOTS = SUB * BK / 8;    // 16-byte slots of a sub-tile
+  static_assert(!DUAL || (!BKN && NB == 2 && SUB_SLOTS % 64 == 0),
+                "a wave's load stays in one sub-tile");
   typedef _Float16 halfx8v __attribute__((ext_vector_type(8)));
   typedef _Float16 halfx4v __attribute__((ext_vector_type(4)));
   typedef short shortx4v __attribute__((ext_vector_type(4)));
@@ -862,7 +872,7 @@ __device__ __forceinline__ void h3_tile(const _Float16* __restrict__ P,
   }
 #pragma unroll
   for (int i = 0; i < B_INST; ++i) {
-    const int q = i * THREADS + wave * 64 + lane;
+    const int q = (i * THREADS + wave * 64) % (DUAL ? SUB_SLOTS : B_INST * THREADS) + lane;
     if constexpr (BKN) {
       // [K x N]: slot q is row q / CPR (one k), position q % CPR of its BNT / 8
       // chunks, holding chunk (q % CPR) ^ swz_h3_kn(row); chunks past N read
@@ -900,6 +910,9 @@ __device__ __forceinline__ void h3_tile(const _Float16* __restrict__ P,
   const auto rb = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<_Float16*>(B + b_first), 0,
       static_cast<int>(bytes_left<_Float16>(static_cast<long long>(N) * K, b_first)), kRsrcWord3);
+  const auto rb2 = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<_Float16*>((DUAL ? B2 : B) + b_first), 0,
+      static_cast<int>(bytes_left<_Float16>(static_cast<long long>(N) * K, b_first)), kRsrcWord3);
 #endif
   auto fetch = [&](_Float16* as, _Float16* bs, int kt) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -912,7 +925,8 @@ __device__ __forceinline__ void h3_tile(const _Float16* __restrict__ P,
                                              0, 0);
 #pragma unroll
     for (int i = 0; i < B_INST; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, bs + 8 * (i * THREADS + wave * 64), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(DUAL && i * THREADS + wave * 64 >= SUB_SLOTS ? rb2 : rb,
+                                               bs + 8 * (i * THREADS + wave * 64), 16,
                                                static_cast<int>(b_off[i]), kt * b_step, 0, 0);
 #endif
   };
@@ -954,7 +968,7 @@ __device__ __forceinline__ void h3_tile(const _Float16* __restrict__ P,
           for (int e = 0; e < 4; ++e) f.b[nb][4 * h + e] = v[e];
         }
       } else {
-        const int r = wn * WN + nb * 32 + li;
+        const int r = DUAL ? nb * SUB + wn * 32 + li : wn * WN + nb * 32 + li;
         f.b[nb] = *reinterpret_cast<const halfx8v*>(bs + r * BK + 8 * (cq ^ swz_rows_h(r)));
       }
     }
@@ -1093,9 +1107,39 @@ __global__ __launch_bounds__(4 * BMT, BMT == 64 ? 2 : 1) void gemm_h3_kernel(
   const int m0 = tm * BMT;
   const int n0 = tn * BNT;
   h3::Acc<BMT, BNT> acc;
-  h3_tile<S, BMT, BNT, BKN, EDGE>(P, B, M, N, K, m0, n0, 0, K / BK, acc);
+  h3_tile<S, BMT, BNT, BKN, EDGE>(P, B, B, M, N, K, m0, n0, 0, K / BK, acc);
   h3_store<BMT, BNT, EDGE>(acc, rscale, M, m0, C + static_cast<long long>(m0) * N + n0, N, M - m0,
                       N - n0);
+}
+
+// SwiGLU of two products against the same planes, act = SiLU(x . W_gate) * (x .
+// W_up): BNT / 2 columns of each per tile, so gate and up never reach memory.
+template <int S, int BMT, int BNT, bool EDGE>
+__global__ __launch_bounds__(4 * BMT, 1) void gemm_h3_glu_kernel(
+    const _Float16* __restrict__ P, const float* __restrict__ rscale,
+    const _Float16* __restrict__ Bg, const _Float16* __restrict__ Bu, float* __restrict__ act, int M,
+    int N, int K, int tiles_m, int tiles_n) {
+  using Sh = h3::Shape<BMT, BNT>;
+  int tm, tn;
+  tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BMT;
+  const int n0 = tn * (BNT / 2);
+  h3::Acc<BMT, BNT> acc;
+  h3_tile<S, BMT, BNT, false, EDGE, true>(P, Bg, Bu, M, N, K, m0, n0, 0, K / BK, acc);
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int lg = lane >> 5;
+  const int col = n0 + (wave % Sh::WGN) * 32 + (lane & 31);
+#pragma unroll
+  for (int mb = 0; mb < Sh::MB; ++mb) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int row = m0 + (wave / Sh::WGN) * Sh::WM + mb * 32 + 8 * (v >> 2) + 4 * lg + (v & 3);
+      const float s = rscale[min(row, M - 1)];
+      if (!EDGE || (row < M && col < N))
+        act[static_cast<long long>(row) * N + col] = swiglu_f32(acc[mb][0][v] * s, acc[mb][1][v] * s);
+    }
+  }
 }
 
 // Stream-K form: workgroups 0 .. dp - 1 compute
@@ -1126,7 +1170,7 @@ __global__ __launch_bounds__(4 * BMT, BMT == 64 ? 2 : 1) void gemm_h3_sk_kernel(
     tile_of(first_tile + static_cast<int>(t), tiles_m, tiles_n, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
-    h3_tile<S, BMT, BNT, BKN, EDGE>(P, B, M, N, K, m0, n0, ka, kb, acc);
+    h3_tile<S, BMT, BNT, BKN, EDGE>(P, B, B, M, N, K, m0, n0, ka, kb, acc);
     if (ka == 0 && kb == plan.nk) {
       h3_store<BMT, BNT, EDGE>(acc, rscale, M, m0, C + static_cast<long long>(m0) * N + n0, N, M - m0,
                           N - n0);
@@ -1278,6 +1322,56 @@ void launch_gemm_h3(const GemmH3Args& a, hipStream_t stream) {
     run(integral_constant<int, 128>{}, integral_constant<int, 256>{}, integral_constant<int, 3>{});
   else
     run(integral_constant<int, 128>{}, integral_constant<int, 128>{}, integral_constant<int, 4>{});
+}
+
+// gemm_h3_glu_kernel where its tiles fill whole rounds of one per CU to 85%: per
+// output column it does the two GEMMs' work without their second launch, the
+// gate / up round trip or the SwiGLU pass, but its tiles are not split by K, so
+// a poorly filled last round goes to the two GEMMs. Tiles of 128 x 64 columns of
+// each matrix, or 128 x 128 where those fill the rounds as well (each plane tile
+// loaded then feeds twice the MFMAs). 512 x 11008 x 4096 (688 tiles of 64
+// columns, 90% of three rounds) 265-270 -> 245-251 us, 1000 rows 517 -> 451, 700
+// x 12000 x 1024 158 -> 129, 2000 x 8192 x 2048 397 -> 352. Output-major weights
+// only: [K x N] sub-tiles ran 5-30% slower than the two GEMMs (512 rows 264 ->
+// 352).
+bool launch_gemm_h3_glu(const GemmH3Args& a, const _Float16* Bu, hipStream_t stream) {
+  ENG_CHECK(gemm_h3_applies(a.M, a.N, a.K, a.B, a.b_kn) &&
+                gemm_h3_applies(a.M, a.N, a.K, Bu, a.b_kn) && aligned_to(a.P, 16) &&
+                a.rscale != nullptr,
+            "matmul (fp16 weights): shape or alignment not supported");
+  if (a.b_kn) return false;
+  const long long cus = device_cu_count();
+  auto tiles = [&](long long bn) { return ((a.M + 127) / 128) * ((a.N + bn - 1) / bn); };
+  auto full = [&](long long bn) {
+    const long long t = tiles(bn);
+    return 100 * t >= 85 * ((t + cus - 1) / cus * cus);
+  };
+  const bool wide = full(128) && tiles(128) >= cus;
+  if (!wide && !(full(64) && tiles(64) >= 2 * cus)) return false;
+  const int M = static_cast<int>(a.M), N = static_cast<int>(a.N), K = static_cast<int>(a.K);
+  auto run = [&](auto bnt, auto stages, auto edge) {
+    constexpr int BNT = decltype(bnt)::value;
+    const int tiles_m = (M + 127) / 128;
+    const int tiles_n = (N + BNT / 2 - 1) / (BNT / 2);
+    const long long ntiles = static_cast<long long>(tiles_m) * tiles_n;
+    ENG_CHECK(ntiles <= 0x7fffffffLL, "matmul: too many tiles for one launch");
+    gemm_h3_glu_kernel<decltype(stages)::value, 128, BNT, decltype(edge)::value>
+        <<<static_cast<unsigned>(ntiles), 512, 0, stream>>>(a.P, a.rscale, a.B, Bu, a.C, M, N, K,
+                                                            tiles_m, tiles_n);
+    ENG_LAUNCH_CHECK();
+  };
+  using std::false_type;
+  using std::integral_constant;
+  using std::true_type;
+  auto pick = [&](auto bnt, auto stages) {
+    const bool whole = M % 128 == 0 && N % (decltype(bnt)::value / 2) == 0;
+    whole ? run(bnt, stages, false_type{}) : run(bnt, stages, true_type{});
+  };
+  if (wide)
+    pick(integral_constant<int, 256>{}, integral_constant<int, 3>{});
+  else
+    pick(integral_constant<int, 128>{}, integral_constant<int, 4>{});
+  return true;
 }
 
 void launch_gemm(const GemmArgs& a, hipStream_t stream) {

@@ -25,6 +25,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "silu.hpp"
 #include "device_sync.hpp"
 
 namespace eng {
@@ -89,12 +90,7 @@ __device__ __forceinline__ float rms_scale(float sumsq, long long K, float eps) 
   return 1.0f / sqrtf(sumsq / static_cast<float>(K) + eps);
 }
 
-// SiLU(g) * u with SiLU(g) = g / (1 + e^-g) (reference src/cpu_ref/swiglu_cpu.cpp:
-// 23-25): fp32 exp and a correctly rounded divide; large negative g gives
-// g / inf = -0, large positive g gives g.
-__device__ __forceinline__ float swiglu_f32(float g, float u) {
-  return g / (1.0f + expf(-g)) * u;
-}
+using eng::swiglu_f32;
 
 // Workgroup id -> logical index so that XCD x (ids x, x + 8, ...) gets a
 // contiguous range of logical indices. A bijection on [0, total).

@@ -516,3 +516,23 @@ def test_ffn_subblock_fused_composition(gpu, stem):
     helpers.assert_within(dout.download(), out64, bound, stem + " fused")
     helpers.assert_within(dout.download(), helpers.expected(c), bound + 2 * U * np.abs(out64),
                           stem + " fused vs golden")
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (500, 11000, 64),     # 128 x 64-column tiles, ragged rows and columns, two K steps
+    (2048, 2048, 96),     # 128 x 128-column tiles, one whole round
+    (1025, 4100, 256),    # ... one row and four columns past a tile
+    (4000, 1000, 32),     # one K step
+])
+def test_rmsnorm_linear_swiglu_one_gemm_over_both_matrices(gpu, orc, M, N, K):
+    """Prompt-sized FFN calls whose gate and up share one GEMM: sampled rows, every
+    tile's last one among them, against the float64 composition."""
+    rng = np.random.default_rng(M + N + K)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    g = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    Wg = (rng.standard_normal((N, K), dtype=np.float32) / np.sqrt(K)).astype(np.float16).view(np.uint16)
+    Wu = (rng.standard_normal((N, K), dtype=np.float32) / np.sqrt(K)).astype(np.float16).view(np.uint16)
+    got = gpu_glu_nk(gpu, x, g, Wg, Wu)
+    rows = np.unique(np.concatenate([np.arange(0, M, 97), np.arange(127, M, 128), [M - 1]]))
+    act64, bd, bs = glu_reference(x[rows], g, np.ascontiguousarray(Wg.T), np.ascontiguousarray(Wu.T))
+    helpers.assert_within(got[rows], act64, np.minimum(bd, bs), f"{M}x{N}x{K}")
