@@ -96,10 +96,13 @@ void stream_delay_async(unsigned microseconds, hipStream_t stream);
 // lease split-K partials) takes level 1, so the inner lease (level 0) never
 // waits on its own caller's lock. The GEMM's stream-K records take level 2:
 // its callers (rmsnorm_linear's normalised rows at level 0, the FFN's
-// buffers at level 1) hold their leases across it.
+// buffers at level 1) hold their leases across it. With `optional` an arena
+// that cannot hold `bytes` (it may not grow under capture, or the allocation
+// fails) gives get() == nullptr instead of an error, for launchers that have a
+// way without scratch.
 class StreamScratch {
  public:
-  StreamScratch(hipStream_t stream, std::size_t bytes, int level = 0);
+  StreamScratch(hipStream_t stream, std::size_t bytes, int level = 0, bool optional = false);
   ~StreamScratch();
   StreamScratch(const StreamScratch&) = delete;
   StreamScratch& operator=(const StreamScratch&) = delete;

@@ -91,7 +91,7 @@ void stream_delay_async(unsigned microseconds, hipStream_t stream) {
   ENG_LAUNCH_CHECK();
 }
 
-StreamScratch::StreamScratch(hipStream_t stream, std::size_t bytes, int level) {
+StreamScratch::StreamScratch(hipStream_t stream, std::size_t bytes, int level, bool optional) {
   ENG_CHECK(level >= 0 && level < kScratchLevels, "stream scratch: no such level");
   int dev = 0;
   ENG_HIP_CHECK(hipGetDevice(&dev));
@@ -113,6 +113,7 @@ StreamScratch::StreamScratch(hipStream_t stream, std::size_t bytes, int level) {
   if (bytes > arena->capacity) {
     // Growing allocates, which a stream under HIP graph capture may not do:
     // the capture needs an arena already sized by the same work run eagerly.
+    if (optional && (query != hipSuccess || cap != hipStreamCaptureStatusNone)) return;
     ENG_HIP_CHECK(query);
     ENG_CHECK(cap == hipStreamCaptureStatusNone,
               "stream scratch: this call needs a larger scratch arena than the capturing "
@@ -122,7 +123,20 @@ StreamScratch::StreamScratch(hipStream_t stream, std::size_t bytes, int level) {
     // blocks below the current one's size in total.)
     const std::size_t want = std::max({bytes, kMinArena, 2 * arena->capacity});
     void* grown = nullptr;
-    ENG_HIP_CHECK(hipMalloc(&grown, want));
+    if (optional) {
+      // This thread may be capturing another stream, which an allocation would
+      // invalidate in any mode but the relaxed one.
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      ENG_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+      const hipError_t err = hipMalloc(&grown, want);
+      ENG_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+      if (err != hipSuccess) {
+        (void)hipGetLastError();  // not left for the next launch check to report
+        return;
+      }
+    } else {
+      ENG_HIP_CHECK(hipMalloc(&grown, want));
+    }
     if (arena->base != nullptr) arena->retired.push_back(arena->base);
     arena->base = grown;
     arena->capacity = want;

@@ -685,13 +685,13 @@ struct Cut {
 // launch and another fill, about 8 us, and 3 more where workgroups cross from
 // one tile into the next.
 Cut cut_of(long long M, long long N, long long nk, long long bm, long long bn, double step,
-           double fill, double rec, long long cus) {
+           double fill, double rec, long long cus, bool may_split) {
   const long long tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   const long long tail = tiles % cus;
   const double round = static_cast<double>(nk) * step + fill;
   Cut c;
   c.us = static_cast<double>((tiles + cus - 1) / cus) * round;
-  if (tail != 0 && nk >= 16 && tiles < 2 * cus) {
+  if (may_split && tail != 0 && nk >= 16 && tiles < 2 * cus) {
     // at least 8 K tiles each
     const long long w = std::max<long long>(tail, std::min(cus, tail * nk / 8));
     const double us = static_cast<double>(tiles / cus) * round + fill +
@@ -702,8 +702,9 @@ Cut cut_of(long long M, long long N, long long nk, long long bm, long long bn, d
   return c;
 }
 
+// False, with nothing launched, if the cut needs records and they cannot be had.
 template <typename C, typename BT, bool BNK>
-void run_split(const GemmArgs& a, Form form, const Cut& cut, long long cus, hipStream_t stream) {
+bool run_split(const GemmArgs& a, Form form, const Cut& cut, long long cus, hipStream_t stream) {
   const int M = static_cast<int>(a.M), N = static_cast<int>(a.N), K = static_cast<int>(a.K);
   const int tiles_m = (M + C::BM - 1) / C::BM;
   const int tiles_n = (N + C::BN - 1) / C::BN;
@@ -733,14 +734,16 @@ void run_split(const GemmArgs& a, Form form, const Cut& cut, long long cus, hipS
   };
   if (tail == 0) {
     go(nullptr);
-    return;
+    return true;
   }
   StreamScratch records(
-      stream, static_cast<std::size_t>(plan.nsk) * 2 * C::BM * C::BN * sizeof(float), 2);
+      stream, static_cast<std::size_t>(plan.nsk) * 2 * C::BM * C::BN * sizeof(float), 2, true);
   float* rec = static_cast<float*>(records.get());
+  if (rec == nullptr) return false;
   go(rec);
   launch_sk_fixup<C::BM, C::BN>(rec, a.C, M, N, tiles_m, tiles_n, static_cast<int>(tail), plan,
                                 stream);
+  return true;
 }
 
 // The tiling of the smallest estimated time. Microseconds per K tile and
@@ -752,7 +755,8 @@ void run_split(const GemmArgs& a, Form form, const Cut& cut, long long cus, hipS
 // against the FP32 instruction's kernels (fp32_us), which stay ahead where one
 // round of their small tiles holds the whole call (1024^3: 17.9 us, 512^3: 5.6).
 template <typename BT, bool BNK>
-bool split_dispatch(const GemmArgs& a, double fp32_us, long long cus, hipStream_t stream) {
+bool split_dispatch(const GemmArgs& a, double fp32_us, long long cus, hipStream_t stream,
+                    bool may_split = true) {
   constexpr int kBVec = 16 / static_cast<int>(sizeof(BT));
   Form form = ALIGNED;
   if (!BNK && a.N % 8 != 0)
@@ -762,21 +766,24 @@ bool split_dispatch(const GemmArgs& a, double fp32_us, long long cus, hipStream_
     form = ANY;
   const long long nk = (a.K + BK - 1) / BK;
   const double part = a.K % BK != 0 ? 1.5 : 0.0;  // the partial K tile, by itself
-  const Cut big = cut_of(a.M, a.N, nk, 256, 128, 2.46, 5.0 + part, 0.05, cus);
-  const Cut mid = cut_of(a.M, a.N, nk, 128, 128, 1.39, 3.5 + part, 0.02, cus);
-  const Cut low = cut_of(a.M, a.N, nk, 128, 64, 0.83, 3.0 + part, 0.01, cus);
-  const Cut sml = cut_of(a.M, a.N, nk, 64, 64, 0.52, 2.0 + part, 0.005, cus);
+  const Cut big = cut_of(a.M, a.N, nk, 256, 128, 2.46, 5.0 + part, 0.05, cus, may_split);
+  const Cut mid = cut_of(a.M, a.N, nk, 128, 128, 1.39, 3.5 + part, 0.02, cus, may_split);
+  const Cut low = cut_of(a.M, a.N, nk, 128, 64, 0.83, 3.0 + part, 0.01, cus, may_split);
+  const Cut sml = cut_of(a.M, a.N, nk, 64, 64, 0.52, 2.0 + part, 0.005, cus, may_split);
   const double best = std::min(std::min(big.us, mid.us), std::min(low.us, sml.us));
   if (fp32_us <= best) return false;
+  bool done = false;
   if (big.us == best)
-    run_split<SplitCfg<256, 128, 4, 2>, BT, BNK>(a, form, big, cus, stream);
+    done = run_split<SplitCfg<256, 128, 4, 2>, BT, BNK>(a, form, big, cus, stream);
   else if (mid.us == best)
-    run_split<SplitCfg<128, 128, 2, 4>, BT, BNK>(a, form, mid, cus, stream);
+    done = run_split<SplitCfg<128, 128, 2, 4>, BT, BNK>(a, form, mid, cus, stream);
   else if (low.us == best)
-    run_split<SplitCfg<128, 64, 2, 2, 2>, BT, BNK>(a, form, low, cus, stream);
+    done = run_split<SplitCfg<128, 64, 2, 2, 2>, BT, BNK>(a, form, low, cus, stream);
   else
-    run_split<SplitCfg<64, 64, 2, 2, 2>, BT, BNK>(a, form, sml, cus, stream);
-  return true;
+    done = run_split<SplitCfg<64, 64, 2, 2, 2>, BT, BNK>(a, form, sml, cus, stream);
+  // Without records (a capturing stream whose arena is too small, or no memory
+  // for it) the call runs on the best cut that needs none.
+  return done || split_dispatch<BT, BNK>(a, fp32_us, cus, stream, false);
 }
 
 }  // namespace

@@ -113,3 +113,37 @@ def test_split_gemm_tiny_values_beside_ordinary_ones(gpu, M, N, K):
     bound = K * U * helpers.absdot(A, B) + U * np.abs(y64) + 2 * K * 2.0**-150
     err = np.abs(got - y64)
     assert (err <= bound).all(), float((err / bound).max())
+
+
+@pytest.mark.parametrize("M,N,K", [(640, 1024, 4096), (1280, 4096, 2048)])
+def test_split_gemm_captured_with_no_eager_call_before(gpu, M, N, K):
+    """Sizes whose K is split over workgroups, captured on a stream with no
+    scratch yet: the call runs on a cut that needs none, as it does for another
+    stream's eager call that cannot disturb the capture."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    y64 = helpers.as_f64(A) @ helpers.as_f64(B)
+    derived, stat = helpers.dot_bounds(helpers.absdot(A, B), y64, K)
+    bound = np.minimum(derived, stat)
+    dA, dB, dC, dE = gpu.upload(A), gpu.upload(B), gpu.empty((M, N), np.float32), gpu.empty((M, N), np.float32)
+    s, other, graph = gpu.stream(), gpu.stream(), None
+    try:
+        graph = gpu.graph(s)
+        with graph:
+            gpu.call("eng_matmul_f32", dA.ptr, dB.ptr, dC.ptr, M, N, K, s.handle)
+            gpu.call("eng_matmul_f32", dA.ptr, dB.ptr, dE.ptr, M, N, K, other.handle)
+        other.sync()
+        eager = dE.download().copy()
+        helpers.assert_within(eager, y64, bound, f"eager {M}x{N}x{K}")
+        for _ in range(3):
+            dC.fill_bytes(0xFF)
+            gpu.sync()
+            graph.launch()
+            s.sync()
+            helpers.assert_within(dC.download(), y64, bound, f"captured {M}x{N}x{K}")
+    finally:
+        if graph is not None:
+            graph.destroy()
+        s.destroy()
+        other.destroy()
