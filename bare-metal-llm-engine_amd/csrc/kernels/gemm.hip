@@ -1184,7 +1184,7 @@ __global__ __launch_bounds__(4 * BMT, BMT == 64 ? 2 : 1) void gemm_h3_sk_kernel(
 }
 
 // The fp16-MFMA form of the fp16-weight GEMM can be switched off
-// (ENGINE_GEMM_NO_H3=1) to compare it with the FP32 MFMA on converted weights.
+// (ENGINE_GEMM_NO_H3=1) to compare it with launch_gemm on the same weights.
 // The 128 x 256 tiles can be switched off (ENGINE_GEMM_H3_NO_WIDE=1).
 bool h3_wide_enabled() {
   static const bool on = [] {
@@ -1333,13 +1333,14 @@ void launch_gemm_h3(const GemmH3Args& a, hipStream_t stream) {
 // columns, 90% of three rounds) 265-270 -> 245-251 us, 1000 rows 517 -> 451, 700
 // x 12000 x 1024 158 -> 129, 2000 x 8192 x 2048 397 -> 352. Output-major weights
 // only: [K x N] sub-tiles ran 5-30% slower than the two GEMMs (512 rows 264 ->
-// 352).
+// 352). Up to 64 rows the GEMMs' 64-row tiles do no work on padding (64 x 32768 x
+// 4096 167 us against 181 here).
 bool launch_gemm_h3_glu(const GemmH3Args& a, const _Float16* Bu, hipStream_t stream) {
   ENG_CHECK(gemm_h3_applies(a.M, a.N, a.K, a.B, a.b_kn) &&
                 gemm_h3_applies(a.M, a.N, a.K, Bu, a.b_kn) && aligned_to(a.P, 16) &&
                 a.rscale != nullptr,
             "matmul (fp16 weights): shape or alignment not supported");
-  if (a.b_kn) return false;
+  if (a.b_kn || a.M <= 64) return false;
   const long long cus = device_cu_count();
   auto tiles = [&](long long bn) { return ((a.M + 127) / 128) * ((a.N + bn - 1) / bn); };
   auto full = [&](long long bn) {
