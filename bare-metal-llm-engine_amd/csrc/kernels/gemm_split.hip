@@ -21,7 +21,7 @@
 // with probabilities down to e^-87, flagged everywhere, 0.88 ms).
 //
 // What bounds it: the matrix cores at the clock the card holds under them
-// (4096^3: matrix cores busy 72% of the cycles at about 1.75 GHz; chains of
+// (4096^3: matrix cores busy 63-72% of the cycles, the clock near 1.75 GHz; chains of
 // this instruction on random registers sustain 1594 TFLOP/s, 266 of these six-
 // product FLOP), then LDS. 4096^3: 908 -> 629 us (151 -> 218 TFLOP/s) against
 // the FP32 instruction, error against float64 1.1e-6 -> 1.0e-6; 512 x 4096 x

@@ -89,7 +89,7 @@ std::size_t gemv_kn_scratch_bytes(const GemvArgs& a, std::int64_t M);
 // when the vector path's requirements fail.
 bool launch_gemv_kn_glu(const GemvArgs& a, const void* Wu, std::int64_t M, hipStream_t stream);
 
-// Few-row linear layers on FP32 MFMA (skinny.hip): y[M x N] = x'[M x K] . W
+// Few-row linear layers on the matrix cores (skinny.hip, few_rows.hip): y[M x N] = x'[M x K] . W
 // (W [K x N]) or x' . W^T (w_nk, W [N x K]), x' = x (or, with rms, x * gamma
 // with row m scaled by 1/sqrt(mean_k x[m][k]^2 + eps) after the sum), W read
 // once for all rows. Rows of one call are independent of each other and of M.
@@ -148,9 +148,8 @@ inline SkinnyArgs skinny_args(const GemvArgs& g, std::int64_t M) {
   return a;
 }
 
-// C[M x N] = A'[M x K] . B[K x N] on FP32 MFMA, where A' = A with column k
-// scaled by gamma_k when gamma is given; with rms, row r of C is further
-// multiplied by 1/sqrt(sum_k A[r][k]^2 / K + eps).
+// C[M x N] = A[M x K] . B[K x N] with fp32 arithmetic: the smallest of the
+// estimates of the kernels of gemm_split.hip and gemm.hip.
 struct GemmArgs {
   const float* A = nullptr;
   const void* B = nullptr;

@@ -8,8 +8,9 @@
 // output-major [N x K] (Y = X . W^T). The reference runs every M > 1 through
 // its register-tiled GEMM (kernels/rmsnorm_linear.cu:195-199,
 // kernels/matmul_register_tiled.cu:176-199); at a few rows a GEMM pads M to
-// its tile and leaves most CUs idle (the MFMA GEMM here: ~114 us at
-// 11008 x 4096 for any M <= 64 against ~15 us to read W once).
+// its tile and leaves most CUs idle (64 x 64 tiles on the FP32 MFMA: ~114 us
+// at 11008 x 4096 for any M <= 64 against ~15 us to read W once).
+// Output-major fp16 W at 5-32 rows goes to few_rows.hip where that applies.
 //
 // Work split (stream-K), shared by both layouts: the work is tiles of 64
 // weight rows (output-major) or columns (reference layout) times units of

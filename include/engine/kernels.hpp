@@ -40,7 +40,7 @@ inline void rmsnorm(const float* in, const float* weight, float* out, std::int64
 }
 
 /// C[M x N] = A[M x K] * B[K x N], row-major, fp32 accumulate; runs on the
-/// FP32 matrix cores (the name is kept from the reference, kernels.hpp:77-81).
+/// matrix cores (the name is kept from the reference, kernels.hpp:77-81).
 inline void matmul_register_tiled(const float* A, const float* B, float* C, std::int64_t M,
                                   std::int64_t N, std::int64_t K, hipStream_t stream = nullptr) {
   ENGINE_ABI_CHECK(eng_matmul_f32(A, B, C, M, N, K, stream));

@@ -223,7 +223,8 @@ int eng_f16_to_f32_host(const eng_half* in, float* out, size_t n);
  *   - rmsnorm_linear with any dimension 0 -> no-op (nothing written)
  * ---------------------------------------------------------------------- */
 
-/* C[M x N] = A[M x K] . B[K x N], fp32 accumulate, on FP32 MFMA.
+/* C[M x N] = A[M x K] . B[K x N], fp32 accumulate: three exact bf16 terms
+ * per value on the bf16 matrix cores, small calls on the FP32 instruction.
  * Replaces engine::cuda::matmul_register_tiled
  * (reference include/engine/kernels.hpp:77-81, kernels/matmul_register_tiled.cu:176-199). */
 int eng_matmul_f32(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K,
@@ -287,7 +288,7 @@ int eng_rmsnorm_linear_f16w_noalloc(const float* in, const float* rms_weight, co
  * Same preconditions, messages and zero-size rules as the reference-layout
  * functions above (K == 0: the GEMVs zero-fill, rmsnorm_linear writes nothing).
  * Each output row is one contiguous stream, so M == 1 needs no split-K
- * reduction; M > 1 runs the FP32 MFMA GEMM with B read as B^T. */
+ * reduction; M > 1 takes the few-row kernels and the GEMMs with B read as B^T. */
 int eng_gemv_f16w_nk(const eng_half* W, const float* x, float* y, int64_t N, int64_t K,
                      eng_stream stream);
 int eng_gemv_f32_nk(const float* W, const float* x, float* y, int64_t N, int64_t K,
