@@ -204,13 +204,18 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void few_rows_nk_kernel(
   // X of block b + 1 and then the pieces of block b + 2 are issued (loads
   // complete in order: waiting for X leaves the younger pieces in flight), then
   // block b is computed. Past the last block the loads read block 0 again.
+  // Only the loop's steps count X loads among those that may still be in flight:
+  // there every set is used by a later step. A set loaded in the last steps may
+  // be used by none, and its loads are then not in the compiled code, so those
+  // steps allow the pieces alone.
   constexpr int XD = MB == 1 ? 2 : 1;  // blocks X is loaded ahead
   [[maybe_unused]] constexpr int XL = 2 * MB + (GAIN ? 2 : 0);
   XSet x0, x1, x2;
   auto step = [&](auto st, XSet& X, XSet& Y, int b, auto masked) {
     using Prev = std::integral_constant<int, (decltype(st)::value + 2) % 3>;
 #if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_s_waitcnt(vmcnt_le(LOADS + (XD - 1) * XL));
+    constexpr int ahead = decltype(masked)::value ? 0 : (XD - 1) * XL;
+    __builtin_amdgcn_s_waitcnt(vmcnt_le(LOADS + ahead));
 #endif
     __builtin_amdgcn_sched_barrier(0);
     barrier_no_fence();

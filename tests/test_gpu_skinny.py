@@ -209,7 +209,7 @@ def test_few_rows_k_zero_and_contracts(gpu):
     (9999, 3080),    # six blocks in the steady loop, then a partial one
     (5000, 1536),    # 32 weight rows per workgroup
     (333, 264),      # 16 weight rows, less than one block
-    (1000, 4104),    # ... eight blocks and 8 values
+    (1000, 4104),    # the two-launch kernel: too few rows per workgroup for this K
 ])
 @pytest.mark.parametrize("M", [5, 16, 17, 32])
 @pytest.mark.parametrize("with_gamma", [True, False])
@@ -231,3 +231,16 @@ def test_few_rows_one_launch_kernel(gpu, orc, M, N, K, with_gamma):
     y = orc.rmsnorm_linear(x, g, W, 1e-5).astype(np.float64)
     derived, stat = helpers.rmsnorm_linear_bounds(x, g, W, y, K)
     helpers.assert_within(dy.download(), y, np.minimum(derived, stat), f"{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("N,K", [
+    (8190, 1288),    # 32 weight rows per workgroup, three blocks, the last partial
+    (4090, 1288),    # 16 rows
+    (9999, 2824),    # 48 rows: after the steady loop three blocks (5-16 rows), six (17-32)
+    (9999, 2056),    # ... two, five
+    (9999, 2048),    # ... one, four
+])
+@pytest.mark.parametrize("M", [16, 32])
+def test_few_rows_one_launch_kernel_tails(gpu, orc, M, N, K):
+    """Every number of blocks past the steady loop, for each workgroup height."""
+    test_few_rows_one_launch_kernel(gpu, orc, M, N, K, True)
