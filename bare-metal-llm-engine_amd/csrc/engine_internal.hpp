@@ -96,10 +96,12 @@ void stream_delay_async(unsigned microseconds, hipStream_t stream);
 // lease split-K partials) takes level 1, so the inner lease (level 0) never
 // waits on its own caller's lock. The GEMM's stream-K records take level 2:
 // its callers (rmsnorm_linear's normalised rows at level 0, the FFN's
-// buffers at level 1) hold their leases across it. With `optional` an arena
-// that cannot hold `bytes` (it may not grow under capture, or the allocation
-// fails) gives get() == nullptr instead of an error, for launchers that have a
-// way without scratch.
+// buffers at level 1) hold their leases across it. With `optional`, for launchers
+// that have a way without scratch, get() == nullptr instead of an error where
+// the arena cannot hold `bytes` (it may not grow under capture, or the allocation
+// fails), and also where another stream or graph could use it at the same time:
+// on hipStreamPerThread, one handle for the streams of all host threads, and in a
+// capture that eng_graph_capture_begin did not begin on this stream.
 class StreamScratch {
  public:
   StreamScratch(hipStream_t stream, std::size_t bytes, int level = 0, bool optional = false);
@@ -115,6 +117,9 @@ class StreamScratch {
 void release_stream_scratch(hipStream_t stream);
 // Clears the "leased during capture" mark of `stream`'s arenas (at capture begin).
 void begin_capture_scratch(hipStream_t stream);
+// Remembers the capture just begun on `stream` as one that ends in
+// adopt_stream_scratch.
+void note_own_capture(hipStream_t stream);
 // Moves the current block of each of `stream`'s arenas that a launch leased
 // while the stream was capturing into `owned`, and gives each such arena a
 // fresh block of its current size. The caller (a captured graph) frees the

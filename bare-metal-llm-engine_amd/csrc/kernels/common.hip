@@ -58,10 +58,27 @@ struct Arena {
 
 constexpr std::size_t kMinArena = std::size_t{1} << 20;
 
-std::mutex g_arenas_mu;  // guards the map, not the arenas
+std::mutex g_arenas_mu;  // guards the maps, not the arenas
 std::map<Key, std::unique_ptr<Arena>>& arenas() {
   static auto* m = new std::map<Key, std::unique_ptr<Arena>>();  // leaked: no exit-time teardown
   return *m;
+}
+// The capture begun last on a stream by eng_graph_capture_begin: its id (a
+// process-wide unique number). An entry outlives its capture, where no other
+// capture has its id.
+std::map<std::pair<int, hipStream_t>, unsigned long long>& own_captures() {
+  static auto* m = new std::map<std::pair<int, hipStream_t>, unsigned long long>();
+  return *m;
+}
+
+// The id of the capture `stream` takes part in; false if it is in none.
+bool capture_id(hipStream_t stream, unsigned long long& id) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status == hipStreamCaptureStatusActive;
 }
 
 }  // namespace
@@ -93,8 +110,27 @@ void stream_delay_async(unsigned microseconds, hipStream_t stream) {
 
 StreamScratch::StreamScratch(hipStream_t stream, std::size_t bytes, int level, bool optional) {
   ENG_CHECK(level >= 0 && level < kScratchLevels, "stream scratch: no such level");
+  // One handle, a stream per host thread: an arena found by it would be shared by
+  // streams that nothing orders.
+  if (optional && stream == hipStreamPerThread) return;
   int dev = 0;
   ENG_HIP_CHECK(hipGetDevice(&dev));
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const hipError_t query = hipStreamIsCapturing(stream, &cap);
+  if (query != hipSuccess) {
+    (void)hipGetLastError();  // not left for the next launch check to report
+    cap = hipStreamCaptureStatusNone;
+  }
+  if (optional && cap != hipStreamCaptureStatusNone) {
+    // Only the end of a capture this library began on this stream hands the
+    // arena's block to the graph: any other graph would keep addressing the block
+    // that the stream's eager calls go on using.
+    unsigned long long id = 0;
+    const bool known = capture_id(stream, id);
+    std::lock_guard<std::mutex> lock(g_arenas_mu);
+    const auto it = own_captures().find({dev, stream});
+    if (!known || it == own_captures().end() || it->second != id) return;
+  }
   Arena* arena = nullptr;
   {
     std::lock_guard<std::mutex> lock(g_arenas_mu);
@@ -103,13 +139,6 @@ StreamScratch::StreamScratch(hipStream_t stream, std::size_t bytes, int level, b
     arena = slot.get();
   }
   std::unique_lock<std::mutex> lock(arena->mu);
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const hipError_t query = hipStreamIsCapturing(stream, &cap);
-  if (query != hipSuccess) {
-    (void)hipGetLastError();  // not left for the next launch check to report
-    cap = hipStreamCaptureStatusNone;
-  }
-  if (cap != hipStreamCaptureStatusNone) arena->captured = true;
   if (bytes > arena->capacity) {
     // Growing allocates, which a stream under HIP graph capture may not do:
     // the capture needs an arena already sized by the same work run eagerly.
@@ -141,6 +170,7 @@ StreamScratch::StreamScratch(hipStream_t stream, std::size_t bytes, int level, b
     arena->base = grown;
     arena->capacity = want;
   }
+  if (cap != hipStreamCaptureStatusNone) arena->captured = true;
   ptr_ = arena->base;
   held_ = lock.release();
 }
@@ -170,6 +200,19 @@ void begin_capture_scratch(hipStream_t stream) {
   }
 }
 
+void note_own_capture(hipStream_t stream) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  unsigned long long id = 0;
+  const bool known = capture_id(stream, id);
+  std::lock_guard<std::mutex> lock(g_arenas_mu);
+  if (known) own_captures()[{dev, stream}] = id;
+  else own_captures().erase({dev, stream});
+}
+
 void adopt_stream_scratch(hipStream_t stream, std::vector<void*>& owned) {
   for (int level = 0; level < kScratchLevels; ++level) {
     Arena* arena = find_arena(stream, level);
@@ -192,6 +235,10 @@ void release_stream_scratch(hipStream_t stream) {
   if (hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();
     return;
+  }
+  {
+    std::lock_guard<std::mutex> lock(g_arenas_mu);
+    own_captures().erase({dev, stream});
   }
   for (int level = 0; level < kScratchLevels; ++level) {
     std::unique_ptr<Arena> arena;

@@ -458,6 +458,7 @@ int eng_graph_capture_begin(eng_stream stream) {
               "eng_graph_capture_begin: capture needs a created stream, not the null stream");
     eng::begin_capture_scratch(eng::as_stream(stream));
     ENG_HIP_CHECK(hipStreamBeginCapture(eng::as_stream(stream), hipStreamCaptureModeThreadLocal));
+    eng::note_own_capture(eng::as_stream(stream));
   });
 }
 

@@ -119,8 +119,13 @@ int eng_check_last_launch(void);
  * (reference include/engine/cuda_stream.hpp:21-124, src/cuda_stream.cpp:11-38).
  * Streams are created at the default priority. eng_stream_destroy waits for
  * the stream's work and releases the stream's scratch arena (the device
- * memory the split-K GEMV, split-KV attention, rmsnorm_linear at M > 1 and the
- * FFN launchers reuse on that stream; it grows to the largest request).
+ * memory the split-K GEMV, split-KV attention, rmsnorm_linear at M > 1, the
+ * FFN launchers and matrix products split by K reuse on that stream; it grows to
+ * the largest request). Arenas are found by (device, stream handle): streams
+ * created elsewhere keep theirs until the process ends, and hipStreamPerThread is
+ * one handle for all host threads, so there calls that need scratch have to be
+ * ordered by the caller (eng_matmul_f32, and the plain FP32 product inside the
+ * other entries, uses no scratch there).
  * ---------------------------------------------------------------------- */
 int eng_stream_create(eng_stream* stream, unsigned int flags);
 int eng_stream_destroy(eng_stream stream);
@@ -162,7 +167,12 @@ int eng_event_elapsed_ms(float* ms, eng_event start, eng_event end);
  * eager calls on the capture stream or with any other graph, may run on any
  * stream, and stays valid after the capture stream is destroyed. Replays of
  * one graph share its blocks: they must not overlap (issue them on one
- * stream, or order them with events). eng_graph_destroy waits for the device
+ * stream, or order them with events). A graph captured with HIP's own calls
+ * takes no blocks over: launchers that need scratch leave the stream's arena in
+ * it, so its replays have to be ordered with that stream's other work and end
+ * before the stream is destroyed. The plain FP32 product (eng_matmul_f32) uses
+ * no scratch in such a capture, nor in one here whose stream's arena is too small
+ * for it, and then sums in another order than its eager call. eng_graph_destroy waits for the device
  * before freeing the graph's blocks.
  * ---------------------------------------------------------------------- */
 typedef void* eng_graph;

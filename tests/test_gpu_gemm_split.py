@@ -7,6 +7,9 @@ instruction.
 
 from __future__ import annotations
 
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -145,5 +148,113 @@ def test_split_gemm_captured_with_no_eager_call_before(gpu, M, N, K):
     finally:
         if graph is not None:
             graph.destroy()
+        s.destroy()
+        other.destroy()
+
+
+class NativeGraph:
+    """A capture of `stream` begun and ended with HIP's own calls."""
+
+    def __init__(self, stream):
+        self.hip = ctypes.CDLL("libamdhip64.so")
+        self.stream = ctypes.c_void_p(stream)
+        self.graph, self.exec = ctypes.c_void_p(0), ctypes.c_void_p(0)
+
+    def ok(self, status):
+        assert status == 0, f"HIP status {status}"
+
+    def __enter__(self):
+        self.ok(self.hip.hipStreamBeginCapture(self.stream, 1))  # thread-local mode
+        return self
+
+    def __exit__(self, *exc):
+        self.ok(self.hip.hipStreamEndCapture(self.stream, ctypes.byref(self.graph)))
+        self.ok(self.hip.hipGraphInstantiate(ctypes.byref(self.exec), self.graph, None, None,
+                                             ctypes.c_size_t(0)))
+
+    def nodes(self):
+        n = ctypes.c_size_t(0)
+        self.ok(self.hip.hipGraphGetNodes(self.graph, None, ctypes.byref(n)))
+        return n.value
+
+    def launch(self, stream):
+        self.ok(self.hip.hipGraphLaunch(self.exec, ctypes.c_void_p(stream)))
+
+    def destroy(self):
+        self.ok(self.hip.hipGraphExecDestroy(self.exec))
+        self.ok(self.hip.hipGraphDestroy(self.graph))
+
+
+def test_split_gemm_in_a_capture_of_the_program_and_on_the_per_thread_stream(gpu):
+    """Sizes whose K is split over workgroups, where no records of their own can be
+    had: in a capture begun with HIP itself, on a stream that has an arena, and on
+    hipStreamPerThread, one handle for every thread's stream. Both run as one
+    launch without records; a capture begun here still has them."""
+    M, N, K = 512, 4096, 4096
+    per_thread = 2  # hipStreamPerThread
+    rng = np.random.default_rng(17)
+    A = [rng.uniform(-1, 1, (M, K)).astype(np.float32) for _ in range(2)]
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    dA, dB = [gpu.upload(a) for a in A], gpu.upload(B)
+    dC = [gpu.empty((M, N), np.float32) for _ in range(2)]
+
+    def call(i, stream):
+        gpu.call("eng_matmul_f32", dA[i].ptr, dB.ptr, dC[i].ptr, M, N, K, stream)
+
+    s, other = gpu.stream(), gpu.stream()
+    native, own = NativeGraph(s.handle), gpu.graph(s)
+    try:
+        call(0, s.handle)
+        s.sync()
+        eager = dC[0].download().copy()
+        y64 = helpers.as_f64(A[0]) @ helpers.as_f64(B)
+        derived, stat = helpers.dot_bounds(helpers.absdot(A[0], B), y64, K)
+        with own:
+            call(0, s.handle)
+        with native:
+            call(0, s.handle)
+        assert native.nodes() == 1
+        for _ in range(3):
+            dC[0].fill_bytes(0xFF)
+            gpu.sync()
+            native.launch(other.handle)
+            call(1, s.handle)  # the stream's eager calls go on meanwhile
+            gpu.sync()
+            one = dC[0].download().copy()
+            helpers.assert_within(one, y64, np.minimum(derived, stat), "replay")
+        own.launch(s)
+        s.sync()
+        assert np.array_equal(dC[0].download(), eager)
+        assert not np.array_equal(eager, one)  # (the split's sums are in another order)
+
+        want = []
+        for i in range(2):
+            with NativeGraph(s.handle) as g:
+                call(i, s.handle)
+            g.launch(s.handle)
+            s.sync()
+            g.destroy()
+            want.append(dC[i].download().copy())
+            dC[i].fill_bytes(0xFF)
+        gpu.sync()
+        done = []
+
+        def work(i):
+            for _ in range(20):
+                call(i, per_thread)
+            gpu.call("eng_stream_sync", per_thread)
+            done.append(i)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert sorted(done) == [0, 1]
+        for i in range(2):
+            assert np.array_equal(dC[i].download(), want[i])
+    finally:
+        native.destroy()
+        own.destroy()
         s.destroy()
         other.destroy()
