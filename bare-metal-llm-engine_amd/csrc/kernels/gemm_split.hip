@@ -7,10 +7,21 @@
 // a1 = bf16(a), a2 = bf16(a - a1), a3 = a - a1 - a2, 8 bits each), products of
 // two bf16 values are exact in fp32, and the sums accumulate in fp32. Of the
 // nine term products six are taken -- (1,1) (1,2) (2,1) (2,2) (1,3) (3,1); the
-// three left out are at most 2^-23 of |a b| together and 1.4e-8 of it in the
-// root mean square, below half an fp32 rounding. An fp16 B is two terms and
-// all six products. So a 16-deep slice takes six roundings of the running sum
-// where the FP32 instruction takes eight.
+// three left out are at most 2^-23 of |a b| together. An fp16 B is two terms and
+// all six products.
+//
+// Each call of the instruction rounds its running sum, and not to the nearest
+// (with all six products on one sum, A . diag(1..2) came out 0.24 x 2^-24 low on
+// average, positive or negative). So the leading products and the five small ones
+// (at most 2^-8 of them) have a running sum each, added at the end: a 16-deep
+// slice rounds the large sum once, where the FP32 instruction rounds it eight
+// times. Error against float64, 2-norms at 4096^3, FP32
+// instruction -> this (in brackets all six products on one sum): U[-1, 1] 1.15e-6
+// -> 3.8e-7 (1.0e-6), U[0, 1] 8.4e-7 -> 3.0e-7 (5.3e-7), half of A zero 8.1e-7 ->
+// 3.2e-7 (9.4e-7), 95% of A zero 2.6e-7 -> 1.0e-7 (4.9e-7). Where one product makes
+// the sum (a diagonal factor) its one rounding, 2.49e-8 and 2^-24 at most, becomes
+// that and the products left out: 2.53e-8, and 1.85 x 2^-24 at most seen, 3 x 2^-24
+// possible.
 //
 // What the split does not hold is found and done again: a value whose third
 // remainder still has bits below bf16's (a value under 2^-110) sets a flag
@@ -24,8 +35,8 @@
 // (4096^3: matrix cores busy 63-72% of the cycles, the clock near 1.75 GHz; chains of
 // this instruction on random registers sustain 1594 TFLOP/s, 266 of these six-
 // product FLOP), then LDS. 4096^3: 908 -> 629 us (151 -> 218 TFLOP/s) against
-// the FP32 instruction, error against float64 1.1e-6 -> 1.0e-6; 512 x 4096 x
-// 4096 120 -> 95 us; 509 x 2051 x 1023 (no row aligned) 64 -> 29.6 us.
+// the FP32 instruction; 512 x 4096 x 4096 120 -> 95 us; 509 x 2051 x 1023 (no row
+// aligned) 64 -> 29.6 us.
 #include "gemm_plan.hpp"
 #include "device_sync.hpp"
 #include "launch.hpp"
@@ -340,12 +351,13 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
       }
     }
   };
+  SplitAcc<C> small;  // the five small products' sum; acc the leading one's
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mb][nb][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) acc[mb][nb][v] = small[mb][nb][v] = 0.0f;
   // MFMAs [lo, hi) of a slice's 6 MB NB, by product, then block.
   constexpr int NM = 6 * MB * NB;
   auto mma = [&](const Slice& f, int lo, int hi) {
@@ -357,34 +369,39 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
           const int n = (i * MB + mb) * NB + nb;
-          if (n >= lo && n < hi)
-            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                f.a[P[i][0]][mb], f.b[P[i][1]][nb], acc[mb][nb], 0, 0, 0);
+          if (n >= lo && n < hi) {
+            floatx16& sum = i == 5 ? acc[mb][nb] : small[mb][nb];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[P[i][0]][mb], f.b[P[i][1]][nb], sum, 0,
+                                                          0, 0);
+          }
         }
     }
   };
 
-  // One K tile per step from stage st: the tile's second slice is read while
-  // the first is multiplied, and the next tile's planes (its values loaded a
-  // step ago) are written to the other stage and the loads of the tile after
-  // it issued meanwhile; one barrier, then the next tile's first slice is read
-  // while the second is multiplied. Past the end the last tile is staged
-  // again, never used. The scheduling groups put each chunk's split (about 50
-  // vector instructions) behind its share of the MFMAs, which leave the vector
-  // unit free for most of their 32 cycles.
+  // One K tile per step from stage st: the first slice is multiplied, the next
+  // tile's planes (its values loaded a step ago) written to the other stage
+  // meanwhile, the loads of the tile after it issued and the tile's second slice
+  // read; one barrier, then the second slice is multiplied and the next tile's
+  // first one read. Each slice is read in the last third of the other's MFMAs,
+  // when the other's small planes are done with: the second sums fit the registers
+  // so (256 x 128 tiles spill outside the loop only; read at the start of the
+  // other's MFMAs they spilled 238 inside, 4096^3 1800 us). Past the end the last
+  // tile is staged again, never used. The scheduling groups put each chunk's split
+  // (about 50 vector instructions) behind its share of the MFMAs, which leave the
+  // vector unit free for most of their 32 cycles.
   [[maybe_unused]] constexpr int READS = 3 * MB + PB * NB * (BNK ? 1 : 2);  // fragment reads of a slice
   Slice x, y;
   auto step = [&](auto st, int next_kt) {
     using Next = std::integral_constant<int, 1 - decltype(st)::value>;
-    read_s(a_stage(st), b_stage(st), 1, y);
     each_chunk([&](auto chc) {
       constexpr int ch = decltype(chc)::value;
+      if constexpr (ch == CH - 1) read_s(a_stage(st), b_stage(st), 1, y);
       put(chc, a_stage(Next{}), b_stage(Next{}), raw[ch], std::true_type{});
       load(chc, next_kt, raw[ch]);
       mma(x, ch * NM / CH, (ch + 1) * NM / CH);
 #if defined(__HIP_DEVICE_COMPILE__)
       constexpr int n = (ch + 1) * NM / CH - ch * NM / CH;
-      constexpr int reads = ch == 0 ? (READS + n - 1) / n : 0;
+      constexpr int reads = ch == CH - 1 ? (READS + n - 1) / n : 0;
 #pragma unroll
       for (int i = 0; i < n; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                             // an MFMA
@@ -397,10 +414,15 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
 #endif
     });
     lds_barrier();
-    read_s(a_stage(Next{}), b_stage(Next{}), 0, x);
-    mma(y, 0, NM);
+    constexpr int H = NM * 2 / 3;
+    mma(y, 0, H);
 #if defined(__HIP_DEVICE_COMPILE__)
-    constexpr int per = (2 * READS + NM - 1) / NM;
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+    read_s(a_stage(Next{}), b_stage(Next{}), 0, x);
+    mma(y, H, NM);
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int per = NM - H > 1 ? (READS + NM - H - 2) / (NM - H - 1) : READS;
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
 #pragma unroll
     for (int i = 0; i < (READS + per - 1) / per; ++i) {
@@ -460,6 +482,10 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
     }
   }
 
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] += small[mb][nb];
   // Non-finite sums (bit 0) and values the three terms do not hold (bit 1).
   bool inf = false;
 #pragma unroll

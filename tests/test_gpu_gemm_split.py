@@ -58,6 +58,42 @@ def test_split_gemm_against_float64(gpu, M, N, K):
     helpers.assert_within(got, y64, np.minimum(derived, stat), f"{M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1536, 4096, 1024),   # 256 x 128 tiles
+    (2048, 2048, 512),    # 128 x 128
+    (509, 2051, 1023),    # 128 x 64 in two K groups
+    (130, 250, 1000),     # 64 x 64 in two K groups
+])
+@pytest.mark.parametrize("kind", ["mixed", "same sign", "half zero", "one product"])
+def test_split_gemm_error_is_that_of_one_rounding_per_slice(gpu, M, N, K, kind):
+    """The leading products' sum is rounded once per 16 k. Independent roundings of
+    a sum that grows to y (in the mean half its square) to 2^-24 of it at most add
+    up to 2^-24 sqrt(K / 32) |y|; all six products on one sum exceed this, as does
+    the FP32 instruction with its eight roundings. A sum of one product is rounded
+    once, 0.42 x 2^-24 in the root mean square, without a bias; the products left
+    out add at most 2 x 2^-24."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    if kind == "same sign":
+        A, B = np.abs(A), np.abs(B)
+    elif kind == "half zero":
+        A = np.maximum(A, 0)
+    elif kind == "one product":
+        n = min(K, N)
+        B = np.zeros((K, N), np.float32)
+        B[np.arange(n), np.arange(n)] = rng.uniform(1, 2, n).astype(np.float32)
+    y64 = helpers.as_f64(A) @ helpers.as_f64(B)
+    err = gemm(gpu, A, B) - y64
+    if kind == "one product":
+        rel = err[:, :n] / np.abs(y64[:, :n]) / U
+        assert np.abs(rel).max() <= 3.1
+        assert np.sqrt((rel * rel).mean()) <= 0.5
+        assert abs(rel.mean()) <= 0.05
+    else:
+        assert np.linalg.norm(err) / np.linalg.norm(y64) <= U * np.sqrt(K / 32)
+
+
 @pytest.mark.parametrize("M,N,K", [(1531, 1024, 1024), (300, 999, 999)])
 def test_split_gemm_times_identity_is_exact(gpu, M, N, K):
     """A . I = A bit for bit: the three terms of a value add up to it, over 200
