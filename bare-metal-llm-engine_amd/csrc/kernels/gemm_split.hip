@@ -165,6 +165,30 @@ __device__ __forceinline__ void load8(const T* p, float (&v)[8]) {
   }
 }
 
+// The same with halves left as they are, in v[0 .. 3]: nothing waits for the load,
+// and it holds four registers until widen8.
+template <bool VEC, typename T>
+__device__ __forceinline__ void load8_raw(const T* p, float (&v)[8]) {
+  if constexpr (std::is_same<T, float>::value) {
+    load8<VEC>(p, v);
+  } else {
+    Half8U h;
+    if constexpr (VEC) h = __builtin_bit_cast(Half8U, *reinterpret_cast<const halfx8*>(p));
+    else h = *reinterpret_cast<const Half8U*>(p);
+    const floatx4 w = __builtin_bit_cast(floatx4, h);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = w[e];
+  }
+}
+template <typename T>
+__device__ __forceinline__ void widen8(float (&v)[8]) {
+  if constexpr (!std::is_same<T, float>::value) {
+    const halfx8 h = __builtin_bit_cast(halfx8, floatx4{v[0], v[1], v[2], v[3]});
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(h[e]);
+  }
+}
+
 // Operand forms. ALIGNED: K % 32 == 0, 16-byte aligned rows, and [K x N] B with N %
 // 8 == 0. ANY: any K and element alignment ([K x N] B: N % 8 == 0). SHIFT: [K x N]
 // B with any N >= 8: the last column chunk of a row, when it crosses N, is
@@ -246,29 +270,40 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
     constexpr int ch = decltype(chc)::value;
     const long long k0 = static_cast<long long>(kt) * BK;
     if constexpr (ch < A8) load8<!GEN>(ap[ch] + k0, v);
-    else load8<!GEN>(bp[ch - A8] + (BNK ? k0 : k0 * N), v);
+    else load8_raw<!GEN>(bp[ch - A8] + (BNK ? k0 : k0 * N), v);
   };
   // The partial K tile, element by element (elements past K are zeros).
   [[maybe_unused]] auto load_partial = [&](auto chc, int kt, float(&v)[8]) {
     constexpr int ch = decltype(chc)::value;
     constexpr bool IS_A = ch < A8;
     constexpr int j = IS_A ? ch : ch - A8;
-    const int q = T * j + t;
+    int q = T * j + t;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(q));  // (its addresses are not kept through the pipeline)
+#endif
     const int k0 = kt * BK;
+    std::conditional_t<IS_A, float, BT> w[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int k = IS_A || BNK ? k0 + 8 * (q & 3) + e : k0 + q / CPR;
-      float w;
-      if constexpr (IS_A) {
-        w = A[static_cast<long long>(min(m0 + (q >> 2), M - 1)) * K + min(k, K - 1)];
-      } else if constexpr (BNK) {
-        w = static_cast<float>(
-            B[static_cast<long long>(min(n0 + (q >> 2), N - 1)) * K + min(k, K - 1)]);
-      } else {
-        w = static_cast<float>(
-            B[static_cast<long long>(min(k, K - 1)) * N + min(n0 + 8 * (q % CPR) + e, N - 1)]);
-      }
-      v[e] = k < K ? w : 0.0f;
+      if constexpr (IS_A)
+        w[e] = A[static_cast<long long>(min(m0 + (q >> 2), M - 1)) * K + min(k, K - 1)];
+      else if constexpr (BNK)
+        w[e] = B[static_cast<long long>(min(n0 + (q >> 2), N - 1)) * K + min(k, K - 1)];
+      else
+        w[e] = B[static_cast<long long>(min(k, K - 1)) * N + min(n0 + 8 * (q % CPR) + e, N - 1)];
+      if (k >= K) w[e] = 0;
+    }
+    if constexpr (std::is_same<std::decay_t<decltype(w[0])>, float>::value) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = w[e];
+    } else {
+      halfx8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = w[e];
+      const floatx4 bits = __builtin_bit_cast(floatx4, h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = bits[e];
     }
   };
   unsigned flag = 0;
@@ -277,6 +312,7 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
     constexpr int ch = decltype(chc)::value;
     constexpr bool IS_A = ch < A8;
     const int q = T * (IS_A ? ch : ch - A8) + t;
+    if constexpr (!IS_A) widen8<BT>(v);
     if constexpr (!IS_A && FORM == SHIFT && decltype(whole)::value) {
 #pragma unroll
       for (int b = 4; b > 0; b >>= 1) {
@@ -358,6 +394,17 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[mb][nb][v] = small[mb][nb][v] = 0.0f;
+  auto fold = [&] {  // the small sums into the large ones
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          acc[mb][nb][v] += small[mb][nb][v];
+          small[mb][nb][v] = 0.0f;
+        }
+  };
   // MFMAs [lo, hi) of a slice's 6 MB NB, by product, then block.
   constexpr int NM = 6 * MB * NB;
   auto mma = [&](const Slice& f, int lo, int hi) {
@@ -459,7 +506,10 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
       step(I1{}, min(first + (i + 3) * KG, last));
     }
     if (i < n) step(I0{}, last);
+    fold();
   }
+  // (the small sums are folded at each tile, so that they hold no registers while
+  // its elements are loaded: 24 loads in flight, not one by one)
 #pragma unroll 1
   for (int k = kt0 + n * KG; k < kt1; k += KG) {
     const int kt = k + group;
@@ -476,16 +526,13 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
     __syncthreads();
     if (kt < kt1) {
       read_s(a_stage(I0{}), b_stage(I0{}), 0, x);
-      read_s(a_stage(I0{}), b_stage(I0{}), 1, y);
       mma(x, 0, NM);
+      read_s(a_stage(I0{}), b_stage(I0{}), 1, y);
       mma(y, 0, NM);
+      fold();
     }
   }
 
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] += small[mb][nb];
   // Non-finite sums (bit 0) and values the three terms do not hold (bit 1).
   bool inf = false;
 #pragma unroll
@@ -641,15 +688,17 @@ template <typename C>
 __device__ __forceinline__ void split_store(const SplitAcc<C>& acc, float* __restrict__ out,
                                             long long ld, int rows_left, int cols_left) {
   if (C::KG > 1 && threadIdx.x >= C::kGroup) return;  // group 0 holds the sum
-  const int lane = threadIdx.x & 63;
+  int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
+#if defined(__HIP_DEVICE_COMPILE__)
+  // keeps the element offsets out of the tile loop's registers (spilled, each was
+  // read back behind the store before: 20 us a tile)
+  asm volatile("" : "+s"(ld), "+v"(lane));
+#endif
   const int li = lane & 31;
   const int lg = lane >> 5;
   const int wm = wave / C::WGN;
   const int wn = wave % C::WGN;
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("" : "+s"(ld));  // keeps the element offsets out of the tile loop's registers
-#endif
   const bool whole = rows_left >= C::BM && cols_left >= C::BN;
 #pragma unroll
   for (int mb = 0; mb < C::MB; ++mb) {
