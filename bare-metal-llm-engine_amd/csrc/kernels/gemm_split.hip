@@ -23,13 +23,16 @@
 // that and the products left out: 2.53e-8, and 1.85 x 2^-24 at most seen, 3 x 2^-24
 // possible.
 //
-// What the split does not hold is found and done again: a value whose third
-// remainder still has bits below bf16's (a value under 2^-110) sets a flag
-// while it is staged, and infinities, NaN and sums past the fp32 range leave a
-// non-finite accumulator. A workgroup that sees the latter, or the former where
-// it could matter next to its sums, recomputes its tile with
-// v_mfma_f32_32x32x2_f32 on the unsplit operands (4096^3 with one NaN 2.3 ms;
-// with probabilities down to e^-87, flagged everywhere, 0.88 ms).
+// What the split does not hold is found and done again on v_mfma_f32_32x32x2_f32
+// with the unsplit operands, element by element (in the 32 x 32 blocks that hold
+// one): sums that are not finite (an infinity, NaN, a sum past the fp32 range), and
+// sums next to which values under 2^-110 could matter, whose third remainder may
+// have bits below bf16's (a flag is set while such a value is staged; then each
+// row's and column's largest magnitudes bound each sum). 4096^3, 630 us, and 900-990
+// on the FP32 instruction alone: one NaN 912 us, NaN in every row 1970,
+// probabilities down to e^-87 everywhere 830, the same with zero columns beside
+// them 834; while one such element had its whole tile done again 2270, 2470, 867
+// and 2770.
 //
 // What bounds it: the matrix cores at the clock the card holds under them
 // (4096^3: matrix cores busy 63-72% of the cycles, the clock near 1.75 GHz; chains of
@@ -533,25 +536,18 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
     }
   }
 
-  // Non-finite sums (bit 0) and values the three terms do not hold (bit 1).
-  bool inf = false;
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) inf |= !(fabsf(acc[mb][nb][v]) <= 3.4028235e38f);
-  const int wave_any = (__ballot(inf) != 0 ? 1 : 0) | (__ballot((flag & 0xffffu) != 0) != 0 ? 2 : 0);
+  // Whether any wave staged a value the three terms do not hold. (After the
+  // barrier every wave has also read its stages.)
+  const bool wave_any = __ballot((flag & 0xffffu) != 0) != 0;
   if (lane == 0) wave_bad[wg_wave] = wave_any;
   __syncthreads();
+  constexpr int W = C::kThreads / 64;
   int any = 0;
 #pragma unroll
-  for (int w = 0; w < C::kThreads / 64; ++w) any |= wave_bad[w];
-  bool again = (any & 1) != 0;
+  for (int w = 0; w < W; ++w) any |= wave_bad[w];
   if constexpr (KG == 2) {
     static_assert(KG * 3 * AP * 2 >= C::BM * C::BN * 4, "the sums fit the A stage");
     float* red = reinterpret_cast<float*>(As0) + wave * (MB * NB * 16 * 64) + lane;
-    // (after the barrier above every wave has read its stages)
     if (group == 1) {
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
@@ -573,30 +569,74 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
   }
   const int k0 = kt0 * BK;
   const int k1 = min(kt1 * BK, K);
-  if (!again && any != 0) {
-    // A value the terms do not hold is off by at most 2^-133, so the sums by
-    // (k1 - k0) 2^-133 (max |a| + max |b|): nothing next to any sum of ordinary
-    // size (tiny probabilities beside large ones), and otherwise again.
-    float amax = 0.0f, bmax = 0.0f, least = 3.4028235e38f;
-    constexpr int W = C::kThreads / 64;
-    // a row's values along k, 8 loads in flight per lane (past the end
-    // the last value again)
-    auto row_max = [&](const auto* row, float m) {
-      for (int k = k0 + lane; k < k1; k += 8 * 64) {
-        float v[8];
+  int li_late = li, lg_late = lg;
+#if defined(__HIP_DEVICE_COMPILE__)
+  // what follows depends on the lane through these, which keeps its addresses out
+  // of the pipeline's registers
+  asm volatile("" : "+v"(li_late), "+v"(lg_late));
+#endif
+  const int lane_late = 32 * lg_late + li_late;
+  // The elements to do again, a bit each: sums that are not finite, and sums that
+  // values the terms do not hold may be off by too much.
+  unsigned again[MB][NB];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = static_cast<float>(row[min(k + 64 * u, k1 - 1)]);
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) m = fmaxf(m, fabsf(v[u]));
+    for (int nb = 0; nb < NB; ++nb) {
+      again[mb][nb] = 0;
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        again[mb][nb] |= fabsf(acc[mb][nb][v]) <= 3.4028235e38f ? 0u : 1u << v;
+    }
+  if (any != 0) {
+    // Such a value is under 2^-110 and off by at most 2^-133, so element (r, c) by
+    // (k1 - k0) 2^-133 (max |B's column c| if row r of A has one + max |A's row r|
+    // if column c of B has one): nothing next to sums of ordinary size (tiny
+    // probabilities beside large ones), and nothing at all where the other factor
+    // is zero. Largest magnitudes per row and column, negative if the row or
+    // column has such a value:
+    float* row_most = reinterpret_cast<float*>(As0);
+    float* col_most = row_most + C::BM;  // BN, or W x BN partial ones
+    static_assert(KG * 3 * AP * 2 >= (C::BM + W * BN) * 4, "the maxima fit the A stage");
+    struct Most {
+      float m = 0.0f;       // the largest magnitude
+      unsigned low = ~0u;   // 2 bits(v) - 2, the least over nonzero v (a zero's wraps)
+      __device__ void add(float v) {
+        m = fmaxf(m, fabsf(v));
+        low = min(low, (__builtin_bit_cast(unsigned, v) << 1) - 2u);
       }
-      return m;
+      __device__ float get() const { return low < 2u * 0x08800000u - 2u ? -m : m; }  // 2^-110
     };
-    for (int r = wg_wave; r < C::BM; r += W)
-      amax = row_max(A + static_cast<long long>(min(m0 + r, M - 1)) * K, amax);
+    auto both = [](float p, float q) {
+      const float n = fmaxf(fabsf(p), fabsf(q));
+      return __builtin_signbit(p) || __builtin_signbit(q) ? -n : n;
+    };
+    // rows along k, four per wave at a time (16 lanes each), 16 loads in flight per
+    // lane (past the end the last value again)
+    auto rows = [&](const auto* base, int first, int end, int count, float* out) {
+      static_assert(C::BM % (4 * W) == 0 && BN % (4 * W) == 0, "whole groups of rows");
+      for (int r0 = 4 * wg_wave; r0 < count; r0 += 4 * W) {
+        const int r = r0 + (lane_late >> 4);
+        const auto* p = base + static_cast<long long>(min(first + r, end)) * K;
+        Most m;
+        for (int k = k0 + (lane_late & 15); k < k1; k += 16 * 16) {
+          float v[16];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) v[u] = static_cast<float>(p[min(k + 16 * u, k1 - 1)]);
+#pragma unroll
+          for (int u = 0; u < 16; ++u) m.add(v[u]);
+        }
+        float x = m.get();
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) x = both(x, __shfl_xor(x, o));
+        if ((lane_late & 15) == 0) out[r] = x;
+      }
+    };
+    rows(A, m0, M - 1, C::BM, row_most);
     if constexpr (BNK) {
-      for (int r = wg_wave; r < BN; r += W)
-        bmax = row_max(B + static_cast<long long>(min(n0 + r, N - 1)) * K, bmax);
+      rows(B, n0, N - 1, BN, col_most);
     } else {
+      Most m[BN / 64];
       for (int k = k0 + 8 * wg_wave; k < k1; k += 8 * W) {
         float v[8][BN / 64];
 #pragma unroll
@@ -604,82 +644,106 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ A, const BT
 #pragma unroll
           for (int c = 0; c < BN / 64; ++c)
             v[u][c] = static_cast<float>(B[static_cast<long long>(min(k + u, k1 - 1)) * N +
-                                           min(n0 + 64 * c + lane, N - 1)]);
+                                           min(n0 + 64 * c + lane_late, N - 1)]);
 #pragma unroll
         for (int u = 0; u < 8; ++u)
 #pragma unroll
-          for (int c = 0; c < BN / 64; ++c) bmax = fmaxf(bmax, fabsf(v[u][c]));
+          for (int c = 0; c < BN / 64; ++c) m[c].add(v[u][c]);
       }
-    }
-    if (group == 0) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) least = fminf(least, fabsf(acc[mb][nb][v]));
-    }
-    float* wave_max = reinterpret_cast<float*>(As0);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      amax = fmaxf(amax, __shfl_xor(amax, o));
-      bmax = fmaxf(bmax, __shfl_xor(bmax, o));
-      least = fminf(least, __shfl_xor(least, o));
-    }
-    if (lane == 0) {
-      wave_max[3 * wg_wave] = amax;
-      wave_max[3 * wg_wave + 1] = bmax;
-      wave_max[3 * wg_wave + 2] = least;
+      for (int c = 0; c < BN / 64; ++c) col_most[wg_wave * BN + 64 * c + lane_late] = m[c].get();
     }
     __syncthreads();
+    if (group == 0) {
+      const float terms = static_cast<float>(k1 - k0);
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      amax = fmaxf(amax, wave_max[3 * w]);
-      bmax = fmaxf(bmax, wave_max[3 * w + 1]);
-      least = fminf(least, wave_max[3 * w + 2]);
-    }
-    // (2^-67 on both sides: 2^-133 is a subnormal)
-    again = !(static_cast<float>(k1 - k0) * 0x1p-66f * (amax + bmax) * 0x1p-40f <= least * 0x1p+1f);
-    __syncthreads();  // As0 is refilled by a following tile
-  }
-  if (again && group == 0) {
-    // Once more on the FP32 instruction, straight from memory.
+      for (int nb = 0; nb < NB; ++nb) {
+        const int c = wn * C::WN + nb * 32 + li_late;
+        float col = col_most[c];
+        if constexpr (!BNK) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[mb][nb][v] = 0.0f;
-    constexpr int U = 8;  // MFMA steps whose loads are in flight together
-#pragma unroll 1
-    for (int k = kt0 * BK; k < k1; k += 2 * U) {
-      float a[U][MB], b[U][NB];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int ku = k + 2 * u + lg;
-        const int kk = min(ku, K - 1);
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          const int r = min(m0 + wm * C::WM + mb * 32 + li, M - 1);
-          const float v = A[static_cast<long long>(r) * K + kk];
-          a[u][mb] = ku < k1 ? v : 0.0f;
+          for (int w = 1; w < W; ++w) col = both(col, col_most[w * BN + c]);
         }
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const int n = min(n0 + wn * C::WN + nb * 32 + li, N - 1);
-          const float v = static_cast<float>(BNK ? B[static_cast<long long>(n) * K + kk]
-                                                 : B[static_cast<long long>(kk) * N + n]);
-          b[u][nb] = ku < k1 ? v : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            acc[mb][nb] =
-                __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][mb], b[u][nb], acc[mb][nb], 0, 0, 0);
+          for (int v = 0; v < 16; ++v) {
+            const float r = row_most[wm * C::WM + mb * 32 + 8 * (v >> 2) + 4 * lg_late + (v & 3)];
+            const float off = (__builtin_signbit(r) ? fabsf(col) * 0x1p-66f : 0.0f) +
+                              (__builtin_signbit(col) ? fabsf(r) * 0x1p-66f : 0.0f);
+            // at most 2^-26 of the sum (both sides times 2^27: 2^-133 is a subnormal)
+            again[mb][nb] |= terms * off * 0x1p-40f <= fabsf(acc[mb][nb][v]) * 2.0f ? 0u : 1u << v;
+          }
+      }
+    }
+    __syncthreads();  // As0 is refilled by a following tile
+  }
+  if (group != 0) return;
+  // Those elements once more, straight from memory on the FP32 instruction, in the
+  // 32 x 32 blocks that hold any: 16 k at a time (lane half lg_late the upper or lower 8
+  // of them), the next ones' loads behind the current ones' MFMAs.
+  constexpr int U = 8;
+  struct Piece {
+    float a[U], b[U];
+  };
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (__ballot(again[mb][nb] != 0) == 0) continue;
+      const float* pa = A + static_cast<long long>(min(m0 + wm * C::WM + mb * 32 + li_late, M - 1)) * K;
+      const int n = min(n0 + wn * C::WN + nb * 32 + li_late, N - 1);
+      const BT* pb = BNK ? B + static_cast<long long>(n) * K : B + n;
+      floatx16 sum;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+      auto load_piece = [&](int k, Piece& f) {
+        load8<false>(pa + k + U * lg_late, f.a);
+        if constexpr (BNK) {
+          load8<false>(pb + k + U * lg_late, f.b);
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            f.b[u] = static_cast<float>(pb[static_cast<long long>(k + U * lg_late + u) * N]);
+        }
+      };
+      auto multiply = [&](const Piece& f) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          sum = __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[u], f.b[u], sum, 0, 0, 0);
+      };
+      Piece f, g;
+      int k = k0;
+      if (k + 2 * U <= k1) {
+        load_piece(k, f);
+#pragma unroll 1
+        for (; k + 6 * U <= k1; k += 4 * U) {
+          load_piece(k + 2 * U, g);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(f);
+          load_piece(k + 4 * U, f);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(g);
+        }
+        multiply(f);
+        k += 2 * U;
+      }
+#pragma unroll 1
+      for (; k < k1; k += 2 * U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int ku = k + U * lg_late + u;
+          const long long kk = min(ku, K - 1);
+          const float va = pa[kk];
+          const float vb = static_cast<float>(pb[BNK ? kk : kk * N]);
+          f.a[u] = ku < k1 ? va : 0.0f;
+          f.b[u] = ku < k1 ? vb : 0.0f;
+        }
+        multiply(f);
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        acc[mb][nb][v] = (again[mb][nb] >> v) & 1u ? sum[v] : acc[mb][nb][v];
     }
   }
 }

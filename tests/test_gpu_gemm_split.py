@@ -154,6 +154,35 @@ def test_split_gemm_tiny_values_beside_ordinary_ones(gpu, M, N, K):
     assert (err <= bound).all(), float((err / bound).max())
 
 
+@pytest.mark.parametrize("M,N,K", [(1536, 4096, 512), (509, 2051, 1023), (300, 999, 4000)])
+def test_split_gemm_recomputes_no_more_than_it_must(gpu, M, N, K):
+    """Infinities and NaN change the elements they reach and no others, bit for bit;
+    neither do exact zeros beside values the three terms do not hold."""
+    rng = np.random.default_rng(23)
+    A = np.exp(-rng.uniform(0, 87, (M, K))).astype(np.float32)
+    A[:, : K // 2] = rng.uniform(-1, 1, (M, K // 2)).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    want = gemm(gpu, A, B)
+    A2, B2 = A.copy(), B.copy()
+    rows, cols = [5, 131, M - 1], [7, 130, N - 1]
+    A2[rows[0], 3], A2[rows[1], K - 1], A2[rows[2], 9] = np.nan, np.inf, -np.inf
+    B2[:, cols] = 0.0
+    zero_rows = [6, 200]
+    A2[zero_rows] = 0.0
+    got = gemm(gpu, A2, B2)
+    keep = np.ones((M, N), bool)
+    keep[rows + zero_rows] = False
+    keep[:, cols] = False
+    assert np.array_equal(got[keep], want[keep])
+    assert (got[zero_rows] == 0).all()
+    ordinary = np.setdiff1d(np.arange(M), rows)
+    assert (got[np.ix_(ordinary, cols)] == 0).all()
+    other = np.setdiff1d(np.arange(N), cols)
+    assert np.isnan(got[rows[0]]).all() and np.isnan(got[np.ix_(rows, cols)]).all()
+    assert np.array_equal(got[rows[1], other], np.sign(B2[K - 1, other]) * np.inf)
+    assert np.array_equal(got[rows[2], other], -np.sign(B2[9, other]) * np.inf)
+
+
 @pytest.mark.parametrize("M,N,K", [(640, 1024, 4096), (1280, 4096, 2048)])
 def test_split_gemm_captured_with_no_eager_call_before(gpu, M, N, K):
     """Sizes whose K is split over workgroups, captured on a stream with no
