@@ -17,13 +17,13 @@
 //     stream kernel over both matrices in one launch and the reduce with the
 //     SwiGLU epilogue (launch_gemv_kn_glu): two launches where the composition
 //     takes five, and the same bits.
+//   * Output-major prefill with fp16 weights, where gemm_h3_glu_applies: the rows
+//     split once into three fp16 planes, then one fp16-MFMA GEMM over both matrices
+//     with SwiGLU in its stores.
 //   * Otherwise gate and up are computed separately into the stream's scratch
 //     arena -- single-row GEMVs, small-batch passes over W, or (more rows)
-//     RMSNorm once and the MFMA GEMM: with fp16 weights (either layout) the
-//     rows are split once into three fp16 planes, and gate and up run either as
-//     one fp16-MFMA GEMM over both with SwiGLU in its stores
-//     (launch_gemm_h3_glu) or each its own (launch_gemm_h3) -- and the SwiGLU
-//     kernel finishes.
+//     RMSNorm once and the MFMA GEMM (fp16 weights, either layout: the planes and
+//     launch_gemm_h3) -- and the SwiGLU kernel finishes.
 // Preconditions and messages follow rmsnorm_linear; any zero dimension
 // writes nothing.
 #include "gemv_kernels.hpp"
@@ -188,6 +188,24 @@ void rmsnorm_linear_swiglu(const float* in, const float* gamma, const WT* Wg, co
     return;
   }
 
+  if (h3 && nk && gemm_h3_glu_applies(M, N)) {
+    const std::size_t plane_bytes =
+        3 * static_cast<std::size_t>(M) * static_cast<std::size_t>(K) * sizeof(_Float16);
+    StreamScratch ws(s, plane_bytes + static_cast<std::size_t>(M) * sizeof(float), 1);
+    GemmH3Args h;
+    h.P = static_cast<const _Float16*>(ws.get());
+    h.rscale = reinterpret_cast<const float*>(static_cast<const char*>(ws.get()) + plane_bytes);
+    h.B = reinterpret_cast<const _Float16*>(Wg);
+    h.C = act;
+    h.M = M;
+    h.N = N;
+    h.K = K;
+    launch_rmsnorm_split3(in, gamma, static_cast<_Float16*>(ws.get()),
+                          const_cast<float*>(h.rscale), M, K, eps, s);
+    launch_gemm_h3_glu(h, reinterpret_cast<const _Float16*>(Wu), s);
+    return;
+  }
+
   const std::size_t mn = static_cast<std::size_t>(M) * static_cast<std::size_t>(N);
   const std::size_t mk = M > 1 ? static_cast<std::size_t>(M) * static_cast<std::size_t>(K) : 0;
   // The leading region holds the normalised rows (4 mk bytes) or the planes
@@ -225,6 +243,10 @@ void rmsnorm_linear_swiglu(const float* in, const float* gamma, const WT* Wg, co
     } else if (!(nk ? launch_gemv_nk_rows(gv, M, s) : launch_gemv_kn_rows(gv, M, s))) {
       // more than a few rows: normalise once, then the MFMA GEMM
       if (h3) {
+        if (!normed) {
+          launch_rmsnorm_split3(in, gamma, planes, rscale, M, K, eps, s);
+          normed = true;
+        }
         GemmH3Args h;
         h.P = planes;
         h.rscale = rscale;
@@ -234,13 +256,6 @@ void rmsnorm_linear_swiglu(const float* in, const float* gamma, const WT* Wg, co
         h.N = N;
         h.K = K;
         h.b_kn = !nk;
-        if (!normed) {
-          launch_rmsnorm_split3(in, gamma, planes, rscale, M, K, eps, s);
-          normed = true;
-          h.C = act;
-          if (launch_gemm_h3_glu(h, reinterpret_cast<const _Float16*>(Wu), s)) return;
-          h.C = out;
-        }
         launch_gemm_h3(h, s);
         continue;
       }

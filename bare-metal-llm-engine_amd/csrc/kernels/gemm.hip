@@ -1335,20 +1335,28 @@ void launch_gemm_h3(const GemmH3Args& a, hipStream_t stream) {
 // only: [K x N] sub-tiles ran 5-30% slower than the two GEMMs (512 rows 264 ->
 // 352). Up to 64 rows the GEMMs' 64-row tiles do no work on padding (64 x 32768 x
 // 4096 167 us against 181 here).
-bool launch_gemm_h3_glu(const GemmH3Args& a, const _Float16* Bu, hipStream_t stream) {
-  ENG_CHECK(gemm_h3_applies(a.M, a.N, a.K, a.B, a.b_kn) &&
-                gemm_h3_applies(a.M, a.N, a.K, Bu, a.b_kn) && aligned_to(a.P, 16) &&
-                a.rscale != nullptr,
-            "matmul (fp16 weights): shape or alignment not supported");
-  if (a.b_kn || a.M <= 64) return false;
+namespace {
+// Columns of each matrix in a tile: 128, 64, or 0 where the two GEMMs are better.
+int h3_glu_columns(std::int64_t M, std::int64_t N) {
+  if (M <= 64) return 0;
   const long long cus = device_cu_count();
-  auto tiles = [&](long long bn) { return ((a.M + 127) / 128) * ((a.N + bn - 1) / bn); };
+  auto tiles = [&](long long bn) { return ((M + 127) / 128) * ((N + bn - 1) / bn); };
   auto full = [&](long long bn) {
     const long long t = tiles(bn);
     return 100 * t >= 85 * ((t + cus - 1) / cus * cus);
   };
-  const bool wide = full(128) && tiles(128) >= cus;
-  if (!wide && !(full(64) && tiles(64) >= 2 * cus)) return false;
+  if (full(128) && tiles(128) >= cus) return 128;
+  return full(64) && tiles(64) >= 2 * cus ? 64 : 0;
+}
+}  // namespace
+
+bool gemm_h3_glu_applies(std::int64_t M, std::int64_t N) { return h3_glu_columns(M, N) != 0; }
+
+void launch_gemm_h3_glu(const GemmH3Args& a, const _Float16* Bu, hipStream_t stream) {
+  const int columns = h3_glu_columns(a.M, a.N);
+  ENG_CHECK(gemm_h3_applies(a.M, a.N, a.K, a.B, false) && gemm_h3_applies(a.M, a.N, a.K, Bu, false) &&
+                !a.b_kn && columns != 0 && aligned_to(a.P, 16) && a.rscale != nullptr,
+            "matmul (fp16 weights): shape or alignment not supported");
   const int M = static_cast<int>(a.M), N = static_cast<int>(a.N), K = static_cast<int>(a.K);
   auto run = [&](auto bnt, auto stages, auto edge) {
     constexpr int BNT = decltype(bnt)::value;
@@ -1368,11 +1376,10 @@ bool launch_gemm_h3_glu(const GemmH3Args& a, const _Float16* Bu, hipStream_t str
     const bool whole = M % 128 == 0 && N % (decltype(bnt)::value / 2) == 0;
     whole ? run(bnt, stages, false_type{}) : run(bnt, stages, true_type{});
   };
-  if (wide)
+  if (columns == 128)
     pick(integral_constant<int, 256>{}, integral_constant<int, 3>{});
   else
     pick(integral_constant<int, 128>{}, integral_constant<int, 4>{});
-  return true;
 }
 
 void launch_gemm(const GemmArgs& a, hipStream_t stream) {

@@ -196,9 +196,11 @@ struct GemmH3Args {
 };
 bool gemm_h3_applies(std::int64_t M, std::int64_t N, std::int64_t K, const void* B, bool b_kn);
 void launch_gemm_h3(const GemmH3Args& a, hipStream_t stream);
-// C = SiLU(x . B) * (x . Bu) for the same planes in one launch. Returns false,
-// launching nothing, where two GEMMs and the SwiGLU pass are the better cut.
-bool launch_gemm_h3_glu(const GemmH3Args& a, const _Float16* Bu, hipStream_t stream);
+// C = SiLU(x . B) * (x . Bu) for the same planes in one launch, B and Bu [N x K]
+// and such as gemm_h3_applies takes; where applies is false two GEMMs and the
+// SwiGLU pass are the better cut.
+bool gemm_h3_glu_applies(std::int64_t M, std::int64_t N);
+void launch_gemm_h3_glu(const GemmH3Args& a, const _Float16* Bu, hipStream_t stream);
 
 // out[i] = SiLU(g[i]) * u[i] in fp32.
 void launch_swiglu_f32(const float* g, const float* u, float* out, long long n,

@@ -536,3 +536,39 @@ def test_rmsnorm_linear_swiglu_one_gemm_over_both_matrices(gpu, orc, M, N, K):
     rows = np.unique(np.concatenate([np.arange(0, M, 97), np.arange(127, M, 128), [M - 1]]))
     act64, bd, bs = glu_reference(x[rows], g, np.ascontiguousarray(Wg.T), np.ascontiguousarray(Wu.T))
     helpers.assert_within(got[rows], act64, np.minimum(bd, bs), f"{M}x{N}x{K}")
+
+
+def test_rmsnorm_linear_swiglu_one_gemm_needs_no_gate_and_up_buffers(gpu):
+    """Captured on a stream whose arena (1 MiB, from a small call) holds the planes of
+    the normalised rows, 0.2 MB, and not gate and up, 44 MB: every replay equals the
+    eager call of another stream."""
+    M, N, K = 500, 11000, 64
+    rng = np.random.default_rng(41)
+    x = gpu.upload(rng.standard_normal((M, K), dtype=np.float32))
+    Wg, Wu = (gpu.upload((rng.standard_normal((N, K), dtype=np.float32) / 8).astype(np.float16).view(np.uint16))
+              for _ in range(2))
+    act = gpu.empty((M, N), np.float32)
+
+    def call(rows, columns, stream):
+        gpu.call("eng_rmsnorm_linear_swiglu_f16w_nk", x.ptr, None, Wg.ptr, Wu.ptr, act.ptr, rows, columns,
+                 K, EPS, stream)
+
+    call(M, N, None)
+    gpu.sync()
+    want = act.download().copy()
+    s, graph = gpu.stream(), None
+    try:
+        call(70, 64, s.handle)
+        graph = gpu.graph(s)
+        with graph:
+            call(M, N, s.handle)
+        for _ in range(3):
+            act.fill_bytes(0xFF)
+            gpu.sync()
+            graph.launch()
+            s.sync()
+            assert np.array_equal(act.download(), want)
+    finally:
+        if graph is not None:
+            graph.destroy()
+        s.destroy()
