@@ -27,6 +27,7 @@
 // (4096 x 11008: 32 against 26.5 us), which is where few_rows_nk_applies draws
 // the line.
 #include "device_sync.hpp"
+#include "gemm_choice.hpp"
 #include "launch.hpp"
 
 #include <algorithm>
@@ -37,8 +38,6 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
-
-constexpr int kBlock16 = 512;  // k of a block (16 waves)
 
 // Maximum of v over the four lanes j, j + 16, j + 32, j + 48, in all of them.
 __device__ __forceinline__ float max4(float v) {
@@ -340,39 +339,9 @@ void run(const SkinnyArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-namespace {
-
-// Estimated microseconds with rt x 16 weight rows per workgroup, at up to 16
-// and 17 to 32 activation rows: per block and round, measured at 11008 x 4096
-// (rt 3), 4096 x 4096 and 4096 x 11008 (rt 1).
-struct Few {
-  int rt = 0;
-  double us16 = 0, us32 = 0;
-};
-Few few_of(long long N, long long K, long long cus) {
-  const double blocks = static_cast<double>((K + kBlock16 - 1) / kBlock16);
-  constexpr double kPer16[3] = {1.35, 1.8, 2.2};
-  constexpr double kPer32[3] = {2.6, 3.0, 3.45};
-  Few best;
-  for (int rt = 1; rt <= 3; ++rt) {
-    const double rounds = static_cast<double>(((N + 16 * rt - 1) / (16 * rt) + cus - 1) / cus);
-    const Few f{rt, 3.2 + rounds * blocks * kPer16[rt - 1], 3.2 + rounds * blocks * kPer32[rt - 1]};
-    if (best.rt == 0 || f.us16 < best.us16) best = f;
-  }
-  return best;
-}
-
-}  // namespace
-
-// Where it is estimated ahead of the stream-K few-row kernel (about 8 us plus
-// the weights at 5 TB/s up to 16 rows, 9 us plus the weights at 3.3 TB/s up to
-// 32) for both row ranges: the choice may not depend on M, whose rows keep
-// their bits.
 bool few_rows_nk_applies(const SkinnyArgs& a) {
-  if (a.w != Elem::F16 || !a.w_nk || !a.rms || a.K > 0x7fffffffLL - kBlock16) return false;
-  const Few f = few_of(a.N, a.K, device_cu_count());
-  const double mb = 2e-6 * static_cast<double>(a.N) * static_cast<double>(a.K);
-  return f.us16 < 8.0 + mb / 5.0 && f.us32 < 9.0 + mb / 3.3;
+  return a.w == Elem::F16 && a.w_nk && a.rms && a.K <= 0x7fffffffLL - kFewBlock &&
+         few_rows_ahead(a.N, a.K, device_cu_count());
 }
 
 void launch_few_rows_nk(const SkinnyArgs& a, hipStream_t stream) {

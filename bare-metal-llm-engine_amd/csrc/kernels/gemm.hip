@@ -27,13 +27,13 @@
 //   * fragments are read a quarter K tile (4 MFMA k-slices) ahead of the MFMAs
 //     that use them.
 // The workgroup -> tile map of every GEMM here is XCD-aware (tile_of).
+#include "gemm_choice.hpp"
 #include "gemm_plan.hpp"
 #include "launch.hpp"
 #include "silu.hpp"
 
 #include <algorithm>
 #include <cstdlib>
-#include <limits>
 #include <type_traits>
 
 namespace eng {
@@ -536,29 +536,6 @@ __global__ __launch_bounds__(f32::kThreads, 2) void gemm_f32_mfma_dma_kernel(
   }
 }
 
-// Direct loads need K % BK == 0, 16-byte aligned operands and 16-byte
-// aligned B rows ([K x N] rows of N elements; [N x K] rows of K), and every
-// lane's byte offset from a tile's corner (up to 64 rows of A, 64 rows of an
-// [N x K] B or BK rows of a [K x N] B) must fit the 31 bits of a buffer
-// load's offset.
-template <bool BNK>
-bool direct_ok(const GemmArgs& a) {
-  constexpr long long kLim = 0x7fffffffLL;
-  const long long b_span = BNK ? static_cast<long long>(f32::BN) * a.K : static_cast<long long>(BK) * a.N;
-  return a.b == Elem::F32 && a.K % BK == 0 && aligned_to(a.A, 16) && aligned_to(a.B, 16) &&
-         (BNK || a.N % 4 == 0) && static_cast<long long>(f32::BM) * a.K * 4 <= kLim &&
-         b_span * 4 <= kLim;
-}
-
-// Estimated time of the 64 x 64 FP32 tiles: per K tile 0.48 us with one
-// workgroup on a CU (1024^3: 256 tiles, 17.9 us) and 0.94 us for a pair (512 x
-// 4096 x 4096: 512 tiles, 120 us).
-double f32_us(const GemmArgs& a, long long cus) {
-  const long long tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  const double nk = static_cast<double>(a.K / BK);
-  return tiles <= cus ? 0.48 * nk : 0.94 * nk * static_cast<double>((tiles + 2 * cus - 1) / (2 * cus));
-}
-
 template <bool BNK>
 void run_gemm_f32(const GemmArgs& a, hipStream_t stream) {
   const int M = static_cast<int>(a.M);
@@ -668,24 +645,6 @@ __global__ __launch_bounds__(256) void gemm_small_splitk_kernel(const float* __r
   }
 }
 
-// 16-byte loads of A and B in the register-staged kernel.
-bool staged_vec(const GemmArgs& a) {
-  const long long vb = a.b == Elem::F32 ? 4 : 8;
-  return a.K % 4 == 0 && aligned_to(a.A, 16) && (a.b_nk ? a.K : a.N) % vb == 0 &&
-         aligned_to(a.B, 16);
-}
-
-// Estimated time of the register-staged kernel: per K tile 0.8 us with one
-// workgroup on a CU and 1.05 us for a pair (1000 x 3000 x 200: 17.5 us), more
-// with element loads (200 x 3001 x 64: 4.8 us; 509 x 2051 x 1023: 64.6 us).
-double staged_us(const GemmArgs& a, long long cus) {
-  const long long tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  const double nk = static_cast<double>((a.K + BK - 1) / BK);
-  const bool vec = staged_vec(a);
-  if (tiles <= cus) return nk * (vec ? 0.8 : a.b == Elem::F32 ? 1.15 : 1.6);
-  return nk * (vec ? 1.05 : 1.9) * static_cast<double>((tiles + 2 * cus - 1) / (2 * cus));
-}
-
 template <typename BT, bool BNK>
 void run_gemm_staged(const GemmArgs& a, hipStream_t stream) {
   const int M = static_cast<int>(a.M);
@@ -697,25 +656,13 @@ void run_gemm_staged(const GemmArgs& a, hipStream_t stream) {
   ENG_CHECK(ntiles <= 0x7fffffffLL, "matmul: too many tiles for one launch");
   const dim3 grid(static_cast<unsigned>(ntiles));
   const BT* B = static_cast<const BT*>(a.B);
-  if (staged_vec(a))
+  if (gemm_staged_vec(gemm_shape(a)))
     gemm_f32_mfma_kernel<BT, BNK, true, true><<<grid, f32::kThreads, 0, stream>>>(
         a.A, B, a.C, M, N, K, tiles_m, tiles_n);
   else
     gemm_f32_mfma_kernel<BT, BNK, false, false><<<grid, f32::kThreads, 0, stream>>>(
         a.A, B, a.C, M, N, K, tiles_m, tiles_n);
   ENG_LAUNCH_CHECK();
-}
-
-bool small_ok(const GemmArgs& a) {
-  return small_enabled() && a.b == Elem::F32 && !a.b_nk && a.M % 32 == 0 && a.N % 32 == 0 &&
-         a.K % 256 == 0 && aligned_to(a.A, 16);
-}
-
-// Estimated time: 0.0065 us per k and round of one 32 x 32 tile per CU (512^3:
-// 5.6 us with about 2.5 of launch; 128 x 4096 x 4096: 63.7 us, two rounds).
-double small_us(const GemmArgs& a, long long cus) {
-  const long long tiles = (a.M / 32) * (a.N / 32);
-  return 0.0065 * static_cast<double>(a.K) * static_cast<double>((tiles + cus - 1) / cus);
 }
 
 void run_gemm_small(const GemmArgs& a, hipStream_t stream) {
@@ -1387,14 +1334,11 @@ void launch_gemm(const GemmArgs& a, hipStream_t stream) {
             "matmul: dimensions must fit in 31 bits");
   // Each kernel's estimate of the call; the smallest runs.
   const long long cus = device_cu_count();
-  const double never = std::numeric_limits<double>::infinity();
-  const bool direct = a.b_nk ? direct_ok<true>(a) : direct_ok<false>(a);
-  const double small = small_ok(a) ? small_us(a, cus) : never;
-  const double f32 = direct ? f32_us(a, cus) : staged_us(a, cus);
-  if (launch_gemm_split(a, std::min(small, f32), cus, stream)) return;
-  if (small <= f32) {
+  const Fp32Choice fp32 = gemm_fp32_choice(gemm_shape(a), cus, small_enabled());
+  if (launch_gemm_split(a, fp32.us, cus, stream)) return;
+  if (fp32.kernel == Fp32Kernel::Small) {
     run_gemm_small(a, stream);
-  } else if (direct) {
+  } else if (fp32.kernel == Fp32Kernel::Direct) {
     a.b_nk ? run_gemm_f32<true>(a, stream) : run_gemm_f32<false>(a, stream);
   } else if (a.b == Elem::F32) {
     a.b_nk ? run_gemm_staged<float, true>(a, stream) : run_gemm_staged<float, false>(a, stream);

@@ -40,6 +40,7 @@
 // product FLOP), then LDS. 4096^3: 908 -> 629 us (151 -> 218 TFLOP/s) against
 // the FP32 instruction; 512 x 4096 x 4096 120 -> 95 us; 509 x 2051 x 1023 (no row
 // aligned) 64 -> 29.6 us.
+#include "gemm_choice.hpp"
 #include "gemm_plan.hpp"
 #include "device_sync.hpp"
 #include "launch.hpp"
@@ -61,7 +62,7 @@ typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 
-constexpr int BK = 32;
+constexpr int BK = kGemmKTile;
 
 // Tile BM x BN by KG groups of WGM x WGN waves; each group takes every KG-th
 // K tile with LDS stages of its own, and the groups' sums are added through
@@ -191,12 +192,6 @@ __device__ __forceinline__ void widen8(float (&v)[8]) {
     for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(h[e]);
   }
 }
-
-// Operand forms. ALIGNED: K % 32 == 0, 16-byte aligned rows, and [K x N] B with N %
-// 8 == 0. ANY: any K and element alignment ([K x N] B: N % 8 == 0). SHIFT: [K x N]
-// B with any N >= 8: the last column chunk of a row, when it crosses N, is
-// read 8 columns before the row's end and shifted into place.
-enum Form { ALIGNED, ANY, SHIFT };
 
 // The K tiles [kt0, kt1) of the tile at (m0, n0) into acc (zeroed here). With
 // two groups only group 0's acc is the sum.
@@ -810,37 +805,6 @@ __global__ __launch_bounds__(C::kThreads, C::kPerCu) void gemm_split_kernel(
   }
 }
 
-// How a call is cut: whole rounds of tiles (one per resident workgroup) run one
-// per workgroup, and the tiles past them either as one more round or, split by
-// K, evenly over up to one workgroup per CU (records and a fix-up pass).
-struct Cut {
-  double us = 0;        // estimated time
-  long long split = 0;  // workgroups sharing the tail tiles (0: not split)
-};
-
-// Estimated time of a tiling: `step` is a workgroup's time per K tile on a full
-// chip, `fill` what a round costs besides (first loads, stores), `rec` what one
-// split workgroup's record adds (written, read back). A split costs the fix-up
-// launch and another fill, about 8 us, and 3 more where workgroups cross from
-// one tile into the next.
-Cut cut_of(long long M, long long N, long long nk, long long bm, long long bn, double step,
-           double fill, double rec, long long cus, bool may_split) {
-  const long long tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-  const long long tail = tiles % cus;
-  const double round = static_cast<double>(nk) * step + fill;
-  Cut c;
-  c.us = static_cast<double>((tiles + cus - 1) / cus) * round;
-  if (may_split && tail != 0 && nk >= 16 && tiles < 2 * cus) {
-    // at least 8 K tiles each
-    const long long w = std::max<long long>(tail, std::min(cus, tail * nk / 8));
-    const double us = static_cast<double>(tiles / cus) * round + fill +
-                      static_cast<double>(tail * nk) / static_cast<double>(w) * step + 8.0 +
-                      rec * static_cast<double>(w) + (w % tail != 0 ? 3.0 : 0.0);
-    if (w > tail && us < c.us) c.us = us, c.split = w;
-  }
-  return c;
-}
-
 // False, with nothing launched, if the cut needs records and they cannot be had.
 template <typename C, typename BT, bool BNK>
 bool run_split(const GemmArgs& a, Form form, const Cut& cut, long long cus, hipStream_t stream) {
@@ -885,43 +849,25 @@ bool run_split(const GemmArgs& a, Form form, const Cut& cut, long long cus, hipS
   return true;
 }
 
-// The tiling of the smallest estimated time. Microseconds per K tile and
-// workgroup, measured with every CU busy (4096^3, 2048^3 and 512 x 4096 x 4096):
-//   256 x 128, 8 waves of 64 x 64                2.46  (4096^3: 629 us, 218 TFLOP/s)
-//   128 x 128, 8 waves of 64 x 32                1.39  (2048^3: 91 us, 189 TFLOP/s)
-//   128 x 64, two groups of 4 waves of 64 x 32   0.83  (512 x 4096 x 4096: 104 us)
-//   64 x 64, two groups of 4 waves of 32 x 32    0.52  (1024^3: 20 us)
-// against the FP32 instruction's kernels (fp32_us), which stay ahead where one
-// round of their small tiles holds the whole call (1024^3: 17.9 us, 512^3: 5.6).
 template <typename BT, bool BNK>
 bool split_dispatch(const GemmArgs& a, double fp32_us, long long cus, hipStream_t stream,
                     bool may_split = true) {
-  constexpr int kBVec = 16 / static_cast<int>(sizeof(BT));
-  Form form = ALIGNED;
-  if (!BNK && a.N % 8 != 0)
-    form = SHIFT;
-  else if (a.K % BK != 0 || !aligned_to(a.A, 16) || !aligned_to(a.B, 16) ||
-           (BNK ? a.K : a.N) % kBVec != 0)
-    form = ANY;
-  const long long nk = (a.K + BK - 1) / BK;
-  const double part = a.K % BK != 0 ? 1.5 : 0.0;  // the partial K tile, by itself
-  const Cut big = cut_of(a.M, a.N, nk, 256, 128, 2.46, 5.0 + part, 0.05, cus, may_split);
-  const Cut mid = cut_of(a.M, a.N, nk, 128, 128, 1.39, 3.5 + part, 0.02, cus, may_split);
-  const Cut low = cut_of(a.M, a.N, nk, 128, 64, 0.83, 3.0 + part, 0.01, cus, may_split);
-  const Cut sml = cut_of(a.M, a.N, nk, 64, 64, 0.52, 2.0 + part, 0.005, cus, may_split);
-  const double best = std::min(std::min(big.us, mid.us), std::min(low.us, sml.us));
-  if (fp32_us <= best) return false;
+  const GemmShape shape = gemm_shape(a);
+  const SplitChoice c = gemm_split_choice(shape, cus, may_split);
+  if (fp32_us <= c.cut.us) return false;
+  const Form form = gemm_split_form(shape);
   bool done = false;
-  if (big.us == best)
-    done = run_split<SplitCfg<256, 128, 4, 2>, BT, BNK>(a, form, big, cus, stream);
-  else if (mid.us == best)
-    done = run_split<SplitCfg<128, 128, 2, 4>, BT, BNK>(a, form, mid, cus, stream);
-  else if (low.us == best)
-    done = run_split<SplitCfg<128, 64, 2, 2, 2>, BT, BNK>(a, form, low, cus, stream);
+  if (c.bm == 256)
+    done = run_split<SplitCfg<256, 128, 4, 2>, BT, BNK>(a, form, c.cut, cus, stream);
+  else if (c.bn == 128)
+    done = run_split<SplitCfg<128, 128, 2, 4>, BT, BNK>(a, form, c.cut, cus, stream);
+  else if (c.bm == 128)
+    done = run_split<SplitCfg<128, 64, 2, 2, 2>, BT, BNK>(a, form, c.cut, cus, stream);
   else
-    done = run_split<SplitCfg<64, 64, 2, 2, 2>, BT, BNK>(a, form, sml, cus, stream);
-  // Without records (a capturing stream whose arena is too small, or no memory
-  // for it) the call runs on the best cut that needs none.
+    done = run_split<SplitCfg<64, 64, 2, 2, 2>, BT, BNK>(a, form, c.cut, cus, stream);
+  // Without records (no memory for them, a capturing stream whose arena is too
+  // small, a stream or capture that may not share it) the call runs on the best
+  // cut that needs none.
   return done || split_dispatch<BT, BNK>(a, fp32_us, cus, stream, false);
 }
 

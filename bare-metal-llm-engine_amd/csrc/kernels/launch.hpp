@@ -4,6 +4,7 @@
 #pragma once
 
 #include "../engine_internal.hpp"
+#include "gemm_choice.hpp"
 
 #include <atomic>
 #include <cstddef>
@@ -161,6 +162,9 @@ struct GemmArgs {
   std::int64_t K = 0;
 };
 void launch_gemm(const GemmArgs& a, hipStream_t stream);
+inline GemmShape gemm_shape(const GemmArgs& a) {
+  return {a.M, a.N, a.K, a.b == Elem::F16, a.b_nk, aligned_to(a.A, 16), aligned_to(a.B, 16)};
+}
 // The same product on the bf16 matrix cores (gemm_split.hip). Returns false,
 // launching nothing, when it estimates more than `fp32_us` microseconds (the
 // caller's own estimate). cus: device_cu_count().

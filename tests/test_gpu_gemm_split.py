@@ -34,20 +34,60 @@ def gemm(gpu, A, B):
     return dC.download()
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (1536, 4096, 512),    # 256 x 128 tiles, whole
-    (1531, 4093, 515),    # ... every edge ragged, a partial K tile, columns shifted into place
-    (2048, 2048, 512),    # 128 x 128
-    (2041, 2056, 530),    # ... ragged, N a multiple of 8
-    (512, 4096, 1000),    # K split over workgroups (records and the fix-up pass)
-    (509, 2051, 1023),    # 128 x 64 in two K groups
-    (130, 250, 1000),     # 64 x 64 in two K groups
-    (129, 257, 993),      # ... one column past a tile, 31 whole K tiles and one value
-    (300, 999, 4000),     # small tiles split over K
-    (4096, 5, 300),       # N below one column chunk
-    (100, 3, 700),
-    (65, 8, 1001),
-])
+# (M, N, K): the tile, operand form and split that a card of 256 CUs gives eng_matmul_f32
+# there (test_gemm_choice.py holds them to the launcher's rules)
+FLOAT64 = {
+    (1536, 4096, 512): "256x128 ALIGNED",
+    (1531, 4093, 515): "256x128 SHIFT",       # every edge ragged, a partial K tile
+    (2041, 2056, 530): "256x128 ANY",
+    (500, 4096, 4096): "256x128 ALIGNED split",  # (records and the fix-up pass)
+    (509, 4090, 4090): "256x128 SHIFT split",
+    (2048, 2048, 512): "128x128 ALIGNED",
+    (2030, 2040, 300): "128x128 ANY",
+    (1000, 4090, 1030): "128x128 SHIFT",
+    (640, 1024, 4096): "128x128 ALIGNED split",
+    (640, 2000, 2050): "128x128 ANY split",
+    (1000, 2050, 1030): "128x128 SHIFT split",
+    (1531, 1024, 1024): "128x64 ALIGNED",     # (two K groups, as in all smaller tiles)
+    (512, 4096, 1000): "128x64 ANY",
+    (509, 2051, 1023): "128x64 SHIFT",
+    (128, 768, 4096): "128x64 ALIGNED split",
+    (128, 1024, 4096): "64x64 ALIGNED split",
+    (65, 8, 1001): "64x64 ANY split",
+    (130, 250, 1000): "64x64 SHIFT split",
+    (129, 257, 993): "64x64 SHIFT split",     # one column past a tile, 31 whole K tiles and one value
+    (300, 999, 4000): "64x64 SHIFT split",
+    (4096, 5, 300): "64x64 SHIFT",            # N below one column chunk
+    (100, 3, 700): "64x64 SHIFT",
+}
+SPECIAL = {
+    (300, 1024, 704): "fp32 direct",
+    (300, 999, 701): "64x64 SHIFT",
+    (300, 512, 4096): "64x64 ALIGNED split",
+    (1531, 1024, 1024): "128x64 ALIGNED",
+    (640, 2000, 2050): "128x128 ANY split",
+    (1536, 4096, 512): "256x128 ALIGNED",
+}
+# M, N, K, weight type, layout of eng_rmsnorm_linear_*
+FORMS = {
+    (1531, 4093, 515, "f32", "nk"): "256x128 ANY",
+    (1531, 4093, 515, "f16", "nk"): "256x128 ANY",
+    (1531, 4093, 515, "f16", "kn"): "256x128 SHIFT",
+    (2030, 2040, 300, "f16", "kn"): "128x128 ANY",
+    (2030, 2041, 300, "f16", "kn"): "128x128 SHIFT",
+    (640, 2000, 2050, "f32", "nk"): "128x128 ANY split",
+    (640, 2000, 2050, "f16", "nk"): "128x128 ANY split",
+    (640, 2000, 2050, "f16", "kn"): "128x128 ANY split",
+    (509, 2051, 1023, "f32", "nk"): "128x64 ANY",
+    (509, 2051, 1023, "f16", "nk"): "128x64 ANY",
+    (509, 2051, 1023, "f16", "kn"): "128x64 SHIFT",
+    (129, 257, 993, "f32", "nk"): "64x64 ANY split",
+    (129, 257, 993, "f16", "nk"): "64x64 ANY split",
+    (129, 257, 993, "f16", "kn"): "64x64 SHIFT split",
+}
+
+
+@pytest.mark.parametrize("M,N,K", FLOAT64)
 def test_split_gemm_against_float64(gpu, M, N, K):
     rng = np.random.default_rng(M + 3 * N + 7 * K)
     A = rng.uniform(-1, 1, (M, K)).astype(np.float32)
@@ -107,7 +147,45 @@ def test_split_gemm_times_identity_is_exact(gpu, M, N, K):
     assert np.array_equal(got[:, :min(K, N)], A[:, :min(K, N)])
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 1024, 704), (300, 999, 701), (1536, 4096, 512)])
+@pytest.mark.parametrize("M,N,K", [(1531, 1024, 1024), (300, 999, 999)])
+def test_split_gemm_subnormal_third_terms_are_exact(gpu, M, N, K):
+    """The smallest values that three terms hold, with third terms (and for the
+    smallest first ones) below bf16's and fp32's normal range: A . I = A bit for bit
+    without a recompute, which the matrix instruction has to keep subnormals for."""
+    rng = np.random.default_rng(7)
+    A = (rng.uniform(1, 2, (M, K)) * 2.0 ** rng.integers(-110, -101, (M, K))).astype(np.float32)
+    A[::2] = (rng.integers(1, 2**16, A[::2].shape) * 2.0**-133).astype(np.float32)
+    A *= rng.choice(np.float32([-1, 1]), A.shape)
+    n = min(K, N)
+    B = np.zeros((K, N), np.float32)
+    B[np.arange(n), np.arange(n)] = 1.0
+    assert np.array_equal(gemm(gpu, A, B)[:, :n], A[:, :n])
+
+
+@pytest.mark.parametrize("M,N,K,w,layout", FORMS)
+def test_split_gemm_weight_types_and_layouts(gpu, M, N, K, w, layout):
+    """fp16 and output-major B at every tile (the normalised rows are the A operand)."""
+    rng = np.random.default_rng(M + N + K)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    W = (0.02 * rng.standard_normal((K, N))).astype(np.float32)
+    if w == "f16":
+        W = W.astype(np.float16).view(np.uint16)
+    dx, dW = gpu.upload(x), gpu.upload(np.ascontiguousarray(W.T) if layout == "nk" else W)
+    dy = gpu.empty((M, N), np.float32)
+    dy.fill_bytes(0xFF)
+    gpu.call(f"eng_rmsnorm_linear_{w}{'w' if w == 'f16' else ''}{'_nk' if layout == 'nk' else ''}",
+             dx.ptr, None, dW.ptr, dy.ptr, M, N, K, 1e-5, None)
+    gpu.sync()
+    x64 = helpers.as_f64(x)
+    y64 = x64 / np.sqrt((x64 * x64).mean(1, keepdims=True) + 1e-5) @ helpers.as_f64(W)
+    got = dy.download()
+    derived, stat = helpers.rmsnorm_linear_bounds(x, None, W, y64, K)
+    helpers.assert_within(got, y64, np.minimum(derived, stat), f"{w} {layout} {M}x{N}x{K}")
+    # one rounding per 16 k, and a few of the row scale
+    assert np.linalg.norm(got - y64) / np.linalg.norm(y64) <= U * (np.sqrt(K / 32) + 8)
+
+
+@pytest.mark.parametrize("M,N,K", SPECIAL)
 def test_split_gemm_infinities_nan_and_extreme_values(gpu, M, N, K):
     rng = np.random.default_rng(11)
     A = rng.uniform(-1, 1, (M, K)).astype(np.float32)
@@ -139,7 +217,7 @@ def test_split_gemm_infinities_nan_and_extreme_values(gpu, M, N, K):
     assert (err <= bound).all(), float((err / bound).max())
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 999, 701), (1536, 4096, 512)])
+@pytest.mark.parametrize("M,N,K", SPECIAL)
 def test_split_gemm_tiny_values_beside_ordinary_ones(gpu, M, N, K):
     """Probabilities down to e^-87 (values the three terms do not hold, in every
     tile) times ordinary values, and rows of nothing but tiny ones."""

@@ -203,14 +203,26 @@ def test_few_rows_k_zero_and_contracts(gpu):
     assert np.all(dy.download() == 7.0)
 
 
-@pytest.mark.parametrize("N,K", [
-    (10000, 520),    # 48 weight rows per workgroup, the last partly past N; a partial k block
-    (8200, 512),     # one whole block
-    (9999, 3080),    # six blocks in the steady loop, then a partial one
-    (5000, 1536),    # 32 weight rows per workgroup
-    (333, 264),      # 16 weight rows, less than one block
-    (1000, 4104),    # the two-launch kernel: too few rows per workgroup for this K
-])
+# (N, K): the kernel and weight rows per workgroup that a card of 256 CUs gives
+# output-major fp16 weights there (test_gemm_choice.py holds them to the rule)
+ONE_LAUNCH = {
+    (10000, 520): "few_rows 48",   # the last rows partly past N; a partial k block
+    (8200, 512): "few_rows 48",    # one whole block
+    (9999, 3080): "few_rows 48",   # six blocks in the steady loop, then a partial one
+    (5000, 1536): "few_rows 32",
+    (333, 264): "few_rows 16",     # less than one block
+    (1000, 4104): "stream-K",      # the two-launch kernel
+}
+ONE_LAUNCH_TAILS = {
+    (8190, 1288): "few_rows 32",   # three blocks, the last partial
+    (4090, 1288): "few_rows 16",
+    (9999, 2824): "few_rows 48",   # past the steady loop three blocks (5-16 rows), six (17-32)
+    (9999, 2056): "few_rows 48",   # ... two, five
+    (9999, 2048): "few_rows 48",   # ... one, four
+}
+
+
+@pytest.mark.parametrize("N,K", ONE_LAUNCH)
 @pytest.mark.parametrize("M", [5, 16, 17, 32])
 @pytest.mark.parametrize("with_gamma", [True, False])
 def test_few_rows_one_launch_kernel(gpu, orc, M, N, K, with_gamma):
@@ -233,13 +245,7 @@ def test_few_rows_one_launch_kernel(gpu, orc, M, N, K, with_gamma):
     helpers.assert_within(dy.download(), y, np.minimum(derived, stat), f"{M}x{N}x{K}")
 
 
-@pytest.mark.parametrize("N,K", [
-    (8190, 1288),    # 32 weight rows per workgroup, three blocks, the last partial
-    (4090, 1288),    # 16 rows
-    (9999, 2824),    # 48 rows: after the steady loop three blocks (5-16 rows), six (17-32)
-    (9999, 2056),    # ... two, five
-    (9999, 2048),    # ... one, four
-])
+@pytest.mark.parametrize("N,K", ONE_LAUNCH_TAILS)
 @pytest.mark.parametrize("M", [16, 32])
 def test_few_rows_one_launch_kernel_tails(gpu, orc, M, N, K):
     """Every number of blocks past the steady loop, for each workgroup height."""
