@@ -21,10 +21,11 @@
 // the same in any batch of 5 to 32 rows.
 //
 // What bounds it: the CU's load path. Each workgroup reads all of X (L2) beside
-// its weights, 256 KiB against 384 KiB at 16 x 11008 x 4096: 20.8 us there
-// (26.2 on the stream-K few-row kernel and its reduce), 18.0 at 5 rows, 30.7 at
-// 32 (36.6); with 16 weight rows per workgroup X outweighs the weights
-// (4096 x 11008: 32 against 26.5 us), which is where few_rows_nk_applies draws
+// its weights, 256 KiB against 384 KiB at 16 x 11008 x 4096: 20.8 us there over
+// three weight buffers (26.2 on the stream-K few-row kernel and its reduce), 18.0
+// at 5 rows, 30.7 at 32 (36.6), and with cold weights 24.0 (26.7), 22.1 (26.1) and
+// 33.8 (36.5); with 16 weight rows per workgroup X outweighs the weights
+// (4096 x 11008: 32 against 26.5 us), which is where few_rows_ahead draws
 // the line.
 #include "device_sync.hpp"
 #include "gemm_choice.hpp"

@@ -1277,7 +1277,7 @@ void launch_gemm_h3(const GemmH3Args& a, hipStream_t stream) {
 // a poorly filled last round goes to the two GEMMs. Tiles of 128 x 64 columns of
 // each matrix, or 128 x 128 where those fill the rounds as well (each plane tile
 // loaded then feeds twice the MFMAs). 512 x 11008 x 4096 (688 tiles of 64
-// columns, 90% of three rounds) 265-270 -> 245-251 us, 1000 rows 517 -> 451, 700
+// columns, 90% of three rounds) 265-270 -> 242-251 us, 1000 rows 517 -> 451, 700
 // x 12000 x 1024 158 -> 129, 2000 x 8192 x 2048 397 -> 352. Output-major weights
 // only: [K x N] sub-tiles ran 5-30% slower than the two GEMMs (512 rows 264 ->
 // 352). Up to 64 rows the GEMMs' 64-row tiles do no work on padding (64 x 32768 x

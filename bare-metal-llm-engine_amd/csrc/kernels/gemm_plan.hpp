@@ -69,7 +69,7 @@ __device__ inline long long sk_worker(long long it, const SkPlan& p) {
 // Split tail tiles: C = the tile's records added in workgroup order. One
 // block per (tail tile, 1024 elements); tiles one workgroup covered whole are
 // skipped (already stored). Bound by the records' read: 512 x 4096 x 4096 in 256
-// x 128 tiles split four ways (33 MB) 11.2 -> 9.7 us with 32-bit plan arithmetic
+// x 128 tiles split four ways (33 MB) 11.2 -> 9 us with 32-bit plan arithmetic
 // and whole groups of record loads in flight.
 template <int BM, int BN, bool EDGE = false>
 __global__ __launch_bounds__(256) void gemm_sk_fixup_kernel(const float* __restrict__ rec,
