@@ -150,6 +150,11 @@ inline SplitChoice gemm_split_choice(const GemmShape& s, long long cus, bool may
   const long long nk = (s.K + kGemmKTile - 1) / kGemmKTile;
   const double part = s.K % kGemmKTile != 0 ? 1.5 : 0.0;  // the partial K tile, by itself
   SplitChoice best;
+  // (the kernel counts k in 32 bits, up to 256 past the end)
+  if (s.K > 0x7fffffffLL - 1024) {
+    best.cut.us = std::numeric_limits<double>::infinity();
+    return best;
+  }
   for (const Tiling& t : kTilings) {
     const Cut c = cut_of(s.M, s.N, nk, t.bm, t.bn, t.step, t.fill + part, t.rec, cus, may_split);
     if (best.bm == 0 || c.us < best.cut.us) best = {t.bm, t.bn, c};

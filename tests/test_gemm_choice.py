@@ -48,3 +48,9 @@ def test_every_tile_and_form_is_among_the_cases():
                          ids=["one launch", "tails"])
 def test_few_row_cases_take_the_kernel_they_name(choose, cases):
     assert dict(zip(cases, choose([f"few {n} {k}" for n, k in cases]))) == cases
+
+
+def test_a_k_that_the_split_kernel_cannot_count_goes_to_the_fp32_instruction(choose):
+    last = 2**31 - 1 - 1024
+    assert choose([f"gemm 17 1 {k} f32 kn" for k in (last, last + 1, 2**31 - 1)]) == [
+        "64x64 SHIFT split", "fp32 staged", "fp32 staged"]
