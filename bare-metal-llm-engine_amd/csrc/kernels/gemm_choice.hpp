@@ -40,9 +40,10 @@ inline double gemm_direct_us(const GemmShape& s, long long cus) {
   return tiles <= cus ? 0.48 * nk : 0.94 * nk * static_cast<double>((tiles + 2 * cus - 1) / (2 * cus));
 }
 
-// 16-byte loads of A and B in the register-staged kernel.
-inline bool gemm_staged_vec(const GemmShape& s) {
-  return s.K % 4 == 0 && s.a16 && (s.b_nk ? s.K : s.N) % (s.half_b ? 8 : 4) == 0 && s.b16;
+// 16-byte loads of A, and of B, in the register-staged kernel.
+inline bool gemm_staged_vec_a(const GemmShape& s) { return s.K % 4 == 0 && s.a16; }
+inline bool gemm_staged_vec_b(const GemmShape& s) {
+  return (s.b_nk ? s.K : s.N) % (s.half_b ? 8 : 4) == 0 && s.b16;
 }
 
 // Estimated time of the register-staged kernel: per K tile 0.8 us with one
@@ -51,7 +52,7 @@ inline bool gemm_staged_vec(const GemmShape& s) {
 inline double gemm_staged_us(const GemmShape& s, long long cus) {
   const long long tiles = ((s.M + 63) / 64) * ((s.N + 63) / 64);
   const double nk = static_cast<double>((s.K + kGemmKTile - 1) / kGemmKTile);
-  const bool vec = gemm_staged_vec(s);
+  const bool vec = gemm_staged_vec_a(s) && gemm_staged_vec_b(s);
   if (tiles <= cus) return nk * (vec ? 0.8 : !s.half_b ? 1.15 : 1.6);
   return nk * (vec ? 1.05 : 1.9) * static_cast<double>((tiles + 2 * cus - 1) / (2 * cus));
 }

@@ -59,6 +59,10 @@ FLOAT64 = {
     (300, 999, 4000): "64x64 SHIFT split",
     (4096, 5, 300): "64x64 SHIFT",            # N below one column chunk
     (100, 3, 700): "64x64 SHIFT",
+    (1000, 3000, 200): "fp32 staged",         # 16-byte loads of both operands,
+    (438, 521, 132): "fp32 staged",           # of A,
+    (300, 336, 85): "fp32 staged",            # of B,
+    (200, 3001, 63): "fp32 staged",           # of neither
 }
 SPECIAL = {
     (300, 1024, 704): "fp32 direct",
