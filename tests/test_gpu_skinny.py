@@ -212,6 +212,8 @@ ONE_LAUNCH = {
     (5000, 1536): "few_rows 32",
     (333, 264): "few_rows 16",     # less than one block
     (1000, 4104): "stream-K",      # the two-launch kernel
+    (8256, 128): "stream-K",       # one unit of k, one launch
+    (8256, 136): "few_rows 48",
 }
 ONE_LAUNCH_TAILS = {
     (8190, 1288): "few_rows 32",   # three blocks, the last partial
