@@ -57,6 +57,8 @@ FLOAT64 = {
     (130, 250, 1000): "64x64 SHIFT split",
     (129, 257, 993): "64x64 SHIFT split",     # one column past a tile, 31 whole K tiles and one value
     (300, 999, 4000): "64x64 SHIFT split",
+    (70, 56, 8190): "64x64 ANY split",        # 32 records to a tile
+    (70, 57, 4100): "64x64 SHIFT split",      # 16
     (4096, 5, 300): "64x64 SHIFT",            # N below one column chunk
     (100, 3, 700): "64x64 SHIFT",
     (1000, 3000, 200): "fp32 staged",         # 16-byte loads of both operands,
