@@ -1003,8 +1003,13 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
   }
 }
 
+// Whether every workgroup takes whole tiles: no records, and nothing left to add.
+bool whole_tiles(const Plan& p) {
+  return p.upt == 1 || (p.U % p.P == 0 && (p.U / p.P) % p.upt == 0);
+}
+
 std::size_t scratch_for(const Plan& p, long long M) {
-  return static_cast<std::size_t>(p.P) * 2 * M * (kCols + 1) * sizeof(float);
+  return whole_tiles(p) ? 0 : static_cast<std::size_t>(p.P) * 2 * M * (kCols + 1) * sizeof(float);
 }
 
 // Output-major fp16 W through LDS stages (WMODE 2) at one m-block, straight
@@ -1032,11 +1037,11 @@ void run_skinny(const SkinnyArgs& a, hipStream_t stream) {
                   " bytes of scratch, more than the " + std::to_string(a.scratch_bytes) +
                   " bytes provided");
     rec = static_cast<float*>(a.scratch);
-  } else {
+  } else if (need != 0) {
     ws = std::make_unique<StreamScratch>(stream, need);
     rec = static_cast<float*>(ws->get());
   }
-  float* rec_ss = rec + plan.P * 2 * static_cast<long long>(M) * kCols;
+  float* rec_ss = rec == nullptr ? nullptr : rec + plan.P * 2 * static_cast<long long>(M) * kCols;
   const unsigned grid = static_cast<unsigned>(plan.P);
   const WT* W = static_cast<const WT*>(a.W);
   if constexpr (NK) {
@@ -1050,8 +1055,7 @@ void run_skinny(const SkinnyArgs& a, hipStream_t stream) {
         W, a.x, a.gamma, a.y, M, N, K, plan, rec, rec_ss, a.eps);
   }
   ENG_LAUNCH_CHECK();
-  // Every workgroup takes whole tiles: nothing left to add.
-  if (plan.U % plan.P == 0 && (plan.U / plan.P) % plan.upt == 0) return;
+  if (whole_tiles(plan)) return;
   skinny_reduce_kernel<RMS><<<dim3(static_cast<unsigned>(plan.tiles), (M + 15) / 16), 256, 0, stream>>>(
       rec, rec_ss, a.y, M, N, K, plan, a.eps);
   ENG_LAUNCH_CHECK();

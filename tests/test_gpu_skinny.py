@@ -252,3 +252,32 @@ def test_few_rows_one_launch_kernel(gpu, orc, M, N, K, with_gamma):
 def test_few_rows_one_launch_kernel_tails(gpu, orc, M, N, K):
     """Every number of blocks past the steady loop, for each workgroup height."""
     test_few_rows_one_launch_kernel(gpu, orc, M, N, K, True)
+
+
+def test_few_rows_of_one_unit_need_no_scratch(gpu, orc):
+    """K within one unit: every workgroup takes whole tiles, so the call leases
+    nothing and can be captured on a stream that has no arena yet (65 weight tiles,
+    and more tiles than workgroups)."""
+    rng = np.random.default_rng(8)
+    K = 128
+    for M, N in ((20, 4130), (8, 33000)):
+        x = rng.standard_normal((M, K), dtype=np.float32)
+        W = orc.f32_to_f16((rng.standard_normal((N, K), dtype=np.float32) / np.sqrt(K)).astype(np.float32))
+        dx, dW, dy = gpu.upload(x), gpu.upload(W), gpu.empty((M, N), np.float32)
+        y = orc.rmsnorm_linear(x, None, np.ascontiguousarray(W.T), 1e-5).astype(np.float64)
+        derived, _ = helpers.rmsnorm_linear_bounds(x, None, np.ascontiguousarray(W.T), y, K)
+        s, graph = gpu.stream(), None
+        try:
+            graph = gpu.graph(s)
+            with graph:
+                gpu.call("eng_rmsnorm_linear_f16w_nk", dx.ptr, None, dW.ptr, dy.ptr, M, N, K, 1e-5, s.handle)
+            for _ in range(3):
+                dy.fill_bytes(0xFF)
+                gpu.sync()
+                graph.launch()
+                s.sync()
+                helpers.assert_within(dy.download(), y, derived, f"{M}x{N}")
+        finally:
+            if graph is not None:
+                graph.destroy()
+            s.destroy()
